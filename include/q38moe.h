@@ -419,6 +419,18 @@ int q38moe_expert_wgrad(const void* G, const void* X, const int32_t* perm, const
                         int32_t k, void* stream);
 
 /*
+ * q38moe_expert_wgrad with a workspace (same arguments and results up to fp32 summation order). Where
+ * E * M * N makes few output tiles and the experts hold many rows (the shared expert as a group of its
+ * own, E = 1), each tile's rows are split over several blocks whose fp32 partial sums go through the
+ * workspace and are added in a fixed order. q38moe_expert_wgrad_workspace_bytes gives its size for
+ * a shape: 0 (workspace may be NULL) where the rows stay whole. Contents need no initialisation.
+ */
+int q38moe_expert_wgrad_workspace_bytes(int64_t T, int32_t M, int32_t N, int32_t E, int32_t k, size_t* bytes);
+int q38moe_expert_wgrad_ws(const void* G, const void* X, const int32_t* perm, const int32_t* starts,
+                           const int32_t* counts, void* dW, int64_t T, int32_t M, int32_t N, int32_t E,
+                           int32_t k, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * SwiGLU backward (act = bf16(silu(g)), h = bf16(act * u), inference.py:378):
  *   d_u = bf16(dh * act), d_g = bf16(bf16(dh * u) * sigmoid(g) * (1 + g * (1 - sigmoid(g))))
  * dH [rows,I], GU = [g | u] [rows,2I], dGU = [d_g | d_u] [rows,2I] bf16; I a multiple of 64.

@@ -747,14 +747,9 @@ int q38moe_transpose_experts(const void* src, void* dst, int32_t E, int32_t R, i
   return Q38MOE_OK;
 }
 
-int q38moe_expert_wgrad(const void* G, const void* X, const int32_t* perm, const int32_t* starts,
-                        const int32_t* counts, void* dW, int64_t T, int32_t M, int32_t N, int32_t E,
-                        int32_t k, void* stream) {
-  g_err[0] = 0;
-  Q38_CHECK(check_routing(T, E, k));
-  Q38_CHECK(check_dim(M, "M"));
-  Q38_CHECK(check_dim(N, "N"));
-  Q38_CHECK(check_ptr(dW, "dW"));
+static int expert_wgrad(const void* G, const void* X, const int32_t* perm, const int32_t* starts,
+                        const int32_t* counts, void* dW, void* partial, int parts, int64_t T, int32_t M, int32_t N,
+                        int32_t E, int32_t k, void* stream) {
   if ((int64_t)E * M * N >= (int64_t)1 << 40) return fail(Q38MOE_EINVAL, "E * M * N is too large");
   if (T > 0) {
     Q38_CHECK(check_rows(T, M > N ? M : N, k));
@@ -765,10 +760,47 @@ int q38moe_expert_wgrad(const void* G, const void* X, const int32_t* perm, const
     return fail(Q38MOE_EINVAL, "starts and counts must not be NULL");
   (void)hipGetLastError();
   Q38_HIP(q38::launch_expert_wgrad(static_cast<const uint16_t*>(G), static_cast<const uint16_t*>(X), perm, starts,
-                                   counts, static_cast<uint16_t*>(dW), T * k, E, M, N, k,
-                                   static_cast<hipStream_t>(stream)),
+                                   counts, static_cast<uint16_t*>(dW), static_cast<float*>(partial), parts, T * k, E,
+                                   M, N, k, static_cast<hipStream_t>(stream)),
           "expert wgrad launch");
   return Q38MOE_OK;
+}
+
+int q38moe_expert_wgrad(const void* G, const void* X, const int32_t* perm, const int32_t* starts,
+                        const int32_t* counts, void* dW, int64_t T, int32_t M, int32_t N, int32_t E,
+                        int32_t k, void* stream) {
+  g_err[0] = 0;
+  Q38_CHECK(check_routing(T, E, k));
+  Q38_CHECK(check_dim(M, "M"));
+  Q38_CHECK(check_dim(N, "N"));
+  Q38_CHECK(check_ptr(dW, "dW"));
+  return expert_wgrad(G, X, perm, starts, counts, dW, nullptr, 1, T, M, N, E, k, stream);
+}
+
+int q38moe_expert_wgrad_workspace_bytes(int64_t T, int32_t M, int32_t N, int32_t E, int32_t k, size_t* bytes) {
+  g_err[0] = 0;
+  Q38_CHECK(check_routing(T, E, k));
+  Q38_CHECK(check_dim(M, "M"));
+  Q38_CHECK(check_dim(N, "N"));
+  if (bytes == nullptr) return fail(Q38MOE_EINVAL, "bytes must not be NULL");
+  const int parts = q38::wgrad_parts(T * k, E, M, N);
+  *bytes = parts > 1 ? sizeof(float) * (size_t)parts * E * M * N : 0;
+  return Q38MOE_OK;
+}
+
+int q38moe_expert_wgrad_ws(const void* G, const void* X, const int32_t* perm, const int32_t* starts,
+                           const int32_t* counts, void* dW, int64_t T, int32_t M, int32_t N, int32_t E, int32_t k,
+                           void* workspace, size_t workspace_bytes, void* stream) {
+  size_t need = 0;
+  Q38_CHECK(q38moe_expert_wgrad_workspace_bytes(T, M, N, E, k, &need));
+  Q38_CHECK(check_ptr(dW, "dW"));
+  if (need > 0) {
+    Q38_CHECK(check_ptr(workspace, "workspace"));
+    if (workspace_bytes < need)
+      return fail(Q38MOE_EWORKSPACE, "workspace holds %zu bytes, %zu needed", workspace_bytes, need);
+  }
+  return expert_wgrad(G, X, perm, starts, counts, dW, workspace, q38::wgrad_parts(T * k, E, M, N), T, M, N, E, k,
+                      stream);
 }
 
 int q38moe_swiglu_backward(const void* dH, const void* GU, void* dGU, int64_t rows, int32_t I,

@@ -211,25 +211,41 @@ __device__ __forceinline__ int wd_off(int row, int col) {
 // indices of slice t into its own LDS ring (global_load_lds_dword, issued two steps before slice
 // t's data copies, which read them), so the pipeline holds no compiler-visible loads: every step
 // issues the same 5 asynchronous copies per wave (4 data + 1 index) and waits with one constant.
-template <bool GX>
+//
+// SPLIT (few tiles: the shared expert as a group of its own has 8 and 4 of them at configuration 2's
+// shapes): nsplit blocks share a tile's rows, block `part` taking slices [part * per, (part + 1) * per)
+// of ceil(slices / nsplit) = per, and store their fp32 sums to partial [nsplit, E, M, N]
+// (zeros where no slice is left), which wgrad_reduce_kernel adds in part order and rounds once.
+template <bool GX, bool SPLIT>
 __global__ __launch_bounds__(512) void expert_wgrad_dma_kernel(const uint16_t* G, const uint16_t* X,
                                                                const int32_t* perm,
                                                                const int32_t* __restrict__ starts,
                                                                const int32_t* __restrict__ counts,
-                                                               uint16_t* __restrict__ dW, int64_t P, int M,
-                                                               int N, int k, int tm, int tn) {
+                                                               uint16_t* __restrict__ dW,
+                                                               float* __restrict__ partial, int64_t P, int M,
+                                                               int N, int k, int tm, int tn, int nsplit) {
   static_assert(!GX || WD_NS == 3, "the index lead below is written for a 3-slot ring");
   __shared__ __align__(16) uint8_t ring_g[WD_NS][WD_BK * 2 * WG_T];   // [slot][row][256 columns]
   __shared__ __align__(16) uint8_t ring_x[WD_NS][WD_BK * 2 * WD_TN];  // [slot][row][256 columns]
   __shared__ __align__(16) int32_t ring_i[GX ? 8 : 1][GX ? 3 : 1][64];  // [wave][slot][row (+32 copies)]
   const int nb = gridDim.x, b = blockIdx.x;
   const int L = (nb & 7) == 0 ? (b & 7) * (nb >> 3) + (b >> 3) : b;
-  const int e = L / (tm * tn), rem = L - e * tm * tn;
+  // Split blocks: a part's tiles side by side, so that they read the same rows at the same time.
+  const int ntiles = SPLIT ? nb / nsplit : nb;
+  const int part = SPLIT ? L / ntiles : 0;
+  const int tile = SPLIT ? L - part * ntiles : L;
+  const int e = tile / (tm * tn), rem = tile - e * tm * tn;
   const int m0 = (rem / tn) * WG_T, n0 = (rem % tn) * WD_TN;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int64_t r0 = P > 0 ? starts[e] : 0;
-  const int cnt = P > 0 ? (int)max((int64_t)0, min((int64_t)counts[e], P - r0)) : 0;
+  int64_t r0 = P > 0 ? starts[e] : 0;
+  int cnt = P > 0 ? (int)max((int64_t)0, min((int64_t)counts[e], P - r0)) : 0;
+  if (SPLIT) {
+    const int per = ((cnt + WD_BK - 1) / WD_BK + nsplit - 1) / nsplit * WD_BK;  // rows per part
+    const int64_t skip = min((int64_t)part * per, (int64_t)cnt);
+    r0 += skip;
+    cnt = (int)min((int64_t)per, (int64_t)cnt - skip);
+  }
   const int nsl = (cnt + WD_BK - 1) / WD_BK;
   // Wave (wm, wn) owns G columns 64 wm .. +63 and X columns 128 wn .. +127 of the tile.
   const int wm = wave >> 1, wn = wave & 1, lr = lane & 31, lh = lane >> 5;
@@ -347,6 +363,24 @@ __global__ __launch_bounds__(512) void expert_wgrad_dma_kernel(const uint16_t* G
   }
 
   // acc[ni][mi][i] of lane l: column n = 128 wn + 32 ni + 8 (i/4) + 4 (l/32) + i%4, row m = 64 wm + 32 mi + l%32.
+  if constexpr (SPLIT) {
+    float* const out = partial + ((int64_t)part * (ntiles / (tm * tn)) + e) * M * N;
+#pragma unroll
+    for (int mi = 0; mi < 2; ++mi) {
+      const int m = m0 + 64 * wm + 32 * mi + lr;
+      if (m >= M) continue;
+#pragma unroll
+      for (int ni = 0; ni < 4; ++ni)
+#pragma unroll
+        for (int gq = 0; gq < 4; ++gq) {
+          const int n = n0 + 128 * wn + 32 * ni + 8 * gq + 4 * lh;
+          if (n < N)
+            *reinterpret_cast<f32x4_t*>(out + (int64_t)m * N + n) =
+                f32x4_t{acc[ni][mi][4 * gq], acc[ni][mi][4 * gq + 1], acc[ni][mi][4 * gq + 2], acc[ni][mi][4 * gq + 3]};
+        }
+    }
+    return;
+  }
   uint16_t* const out = dW + (int64_t)e * M * N;
 #pragma unroll
   for (int mi = 0; mi < 2; ++mi) {
@@ -363,6 +397,32 @@ __global__ __launch_bounds__(512) void expert_wgrad_dma_kernel(const uint16_t* G
                          pack_bf16x2(acc[ni][mi][4 * gq + 2], acc[ni][mi][4 * gq + 3]));
       }
   }
+}
+
+// dW[i] = bf16(sum over the parts, in order, of partial[part][i]); four elements per thread. The parts'
+// loads are independent and issued eight at a time.
+__global__ __launch_bounds__(256) void wgrad_reduce_kernel(const float* __restrict__ partial,
+                                                           uint16_t* __restrict__ dW, int64_t n4, int nsplit) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n4) return;
+  const f32x4_t* src = reinterpret_cast<const f32x4_t*>(partial) + i;
+  f32x4_t s = src[0];
+  int p = 1;
+  for (; p + 8 <= nsplit; p += 8) {
+    f32x4_t v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = src[(int64_t)(p + j) * n4];
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) s[c] += v[j][c];
+  }
+  for (; p < nsplit; ++p) {
+    const f32x4_t v = src[(int64_t)p * n4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) s[c] += v[c];
+  }
+  reinterpret_cast<uint2*>(dW)[i] = make_uint2(pack_bf16x2(s[0], s[1]), pack_bf16x2(s[2], s[3]));
 }
 
 // 8 x 8 transpose of 16-bit elements held as 8 rows of 16 bytes: b[j] = column j of a.
@@ -446,20 +506,45 @@ hipError_t launch_gather_rows(const uint16_t* src, const int32_t* perm, const ui
   return hipGetLastError();
 }
 
+// Parts each tile's rows are split into. One block per CU walks a tile's rows at about 0.9 us per
+// 32-row slice, so few tiles over many rows leave the chip idle. Parts fill the CUs once, of at
+// least 8 slices each: below that the parts' prologues and their fp32 partial sums (M * N * 4 bytes
+// each, written and read back) cost more than the shorter walk gains. Tiles that fill half the CUs or
+// more stay whole: two parts would then add a partial round of blocks and the reduction. At
+// T = 16384, h = 1024, I = 256 the shared expert's gradients (E = 1, 8 and 4 tiles) took 460 and
+// 420 us whole and take 35 + 11 and 27 + 11 us in 32 and 64 parts.
+int wgrad_parts(int64_t P, int E, int M, int N) {
+  const int64_t tiles = (int64_t)E * ((M + WG_T - 1) / WG_T) * ((N + WD_TN - 1) / WD_TN);
+  const int64_t by_cus = device_cus() / (tiles > 0 ? tiles : 1);
+  const int64_t by_rows = P / (E > 0 ? E : 1) / (8 * WD_BK);
+  const int64_t parts = by_cus < by_rows ? by_cus : by_rows;
+  return parts < 2 ? 1 : (int)parts;
+}
+
 hipError_t launch_expert_wgrad(const uint16_t* G, const uint16_t* X, const int32_t* perm, const int32_t* starts,
-                               const int32_t* counts, uint16_t* dW, int64_t P, int E, int M, int N, int k,
-                               hipStream_t stream) {
-  const int tm = (M + WG_T - 1) / WG_T, tn = (N + WG_T - 1) / WG_T;
+                               const int32_t* counts, uint16_t* dW, float* partial, int parts, int64_t P, int E,
+                               int M, int N, int k, hipStream_t stream) {
+  const int tm = (M + WG_T - 1) / WG_T, tn = (N + WD_TN - 1) / WD_TN;
   const int64_t nb = (int64_t)E * tm * tn;
   if (nb == 0) return hipSuccess;
-  const int tnd = (N + WD_TN - 1) / WD_TN;
-  const dim3 grid((unsigned)((int64_t)E * tm * tnd));
-  if (perm == nullptr)
-    hipLaunchKernelGGL(expert_wgrad_dma_kernel<false>, grid, dim3(512), 0, stream, G, X, perm, starts, counts, dW, P,
-                       M, N, k, tm, tnd);
-  else
-    hipLaunchKernelGGL(expert_wgrad_dma_kernel<true>, grid, dim3(512), 0, stream, G, X, perm, starts, counts, dW, P,
-                       M, N, k, tm, tnd);
+  if (parts < 1) return hipErrorInvalidValue;
+  const dim3 grid((unsigned)(nb * parts));
+#define Q38_WGRAD(GX, SPLIT)                                                                                     \
+  hipLaunchKernelGGL((expert_wgrad_dma_kernel<GX, SPLIT>), grid, dim3(512), 0, stream, G, X, perm, starts, counts, \
+                     dW, partial, P, M, N, k, tm, tn, parts)
+  if (parts == 1) {
+    if (perm == nullptr) Q38_WGRAD(false, false);
+    else Q38_WGRAD(true, false);
+    return hipGetLastError();
+  }
+  if (perm == nullptr) Q38_WGRAD(false, true);
+  else Q38_WGRAD(true, true);
+#undef Q38_WGRAD
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  const int64_t n4 = (int64_t)E * M * N / 4;
+  hipLaunchKernelGGL(wgrad_reduce_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, stream, partial, dW, n4,
+                     parts);
   return hipGetLastError();
 }
 

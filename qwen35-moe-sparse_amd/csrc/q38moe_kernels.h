@@ -142,10 +142,12 @@ hipError_t launch_gather_rows(const uint16_t* src, const int32_t* perm, const ui
 // dst[e] = src[e]^T, bf16 [E, R, C] -> [E, C, R]; R, C multiples of 64.
 hipError_t launch_transpose_experts(const uint16_t* src, uint16_t* dst, int E, int R, int C, hipStream_t stream);
 // dW[e] = G_e^T . X_e over each expert's sorted rows (X gathered through perm / k, or sorted rows
-// when perm is NULL); G [P, M], dW [E, M, N] bf16.
+// when perm is NULL); G [P, M], dW [E, M, N] bf16. With parts > 1 (wgrad_parts says how many pay) each
+// tile's rows are split over that many blocks through partial, fp32 [parts, E, M, N].
+int wgrad_parts(int64_t P, int E, int M, int N);
 hipError_t launch_expert_wgrad(const uint16_t* G, const uint16_t* X, const int32_t* perm, const int32_t* starts,
-                               const int32_t* counts, uint16_t* dW, int64_t P, int E, int M, int N, int k,
-                               hipStream_t stream);
+                               const int32_t* counts, uint16_t* dW, float* partial, int parts, int64_t P, int E,
+                               int M, int N, int k, hipStream_t stream);
 hipError_t launch_swiglu_backward(const uint16_t* dH, const uint16_t* GU, uint16_t* dGU, int64_t rows, int I,
                                   hipStream_t stream);
 

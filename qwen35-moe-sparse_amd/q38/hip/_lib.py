@@ -67,6 +67,9 @@ SIGNATURES = {
     "q38moe_gather_rows": (_c_int, [_vp] * 6 + [_c_i64, _c_i32, _c_i32, _c_i32, _vp]),
     "q38moe_transpose_experts": (_c_int, [_vp, _vp, _c_i32, _c_i32, _c_i32, _vp]),
     "q38moe_expert_wgrad": (_c_int, [_vp] * 6 + [_c_i64, _c_i32, _c_i32, _c_i32, _c_i32, _vp]),
+    "q38moe_expert_wgrad_workspace_bytes": (_c_int, [_c_i64, _c_i32, _c_i32, _c_i32, _c_i32,
+                                                     ctypes.POINTER(_c_size)]),
+    "q38moe_expert_wgrad_ws": (_c_int, [_vp] * 6 + [_c_i64, _c_i32, _c_i32, _c_i32, _c_i32, _vp, _c_size, _vp]),
     "q38moe_swiglu_backward": (_c_int, [_vp, _vp, _vp, _c_i64, _c_i32, _vp]),
 }
 

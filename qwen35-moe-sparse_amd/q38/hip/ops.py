@@ -369,8 +369,17 @@ def expert_wgrad(G, X, starts, counts, k, perm=None):
         raise ValueError("without perm, X must hold the G's sorted rows")
     T = P // k
     dW = torch.empty(E, M, N, dtype=torch.bfloat16, device=G.device)
-    check(lib.q38moe_expert_wgrad(_ptr(G), _ptr(X), _ptr(perm), _ptr(starts), _ptr(counts), _ptr(dW), T, M, N, E, k,
-                                  _stream(G.device)), "q38moe_expert_wgrad")
+    ws, n = None, ctypes.c_size_t()
+    if E * M * N <= 128 * 256 * 256:  # rows are split only where 256 x 256 tiles fill at most half the CUs
+        check(lib.q38moe_expert_wgrad_workspace_bytes(T, M, N, E, k, ctypes.byref(n)),
+              "q38moe_expert_wgrad_workspace_bytes")
+    if n.value:
+        ws = torch.empty(n.value, dtype=torch.uint8, device=G.device)
+        check(lib.q38moe_expert_wgrad_ws(_ptr(G), _ptr(X), _ptr(perm), _ptr(starts), _ptr(counts), _ptr(dW), T, M, N,
+                                         E, k, _ptr(ws), n.value, _stream(G.device)), "q38moe_expert_wgrad_ws")
+    else:
+        check(lib.q38moe_expert_wgrad(_ptr(G), _ptr(X), _ptr(perm), _ptr(starts), _ptr(counts), _ptr(dW), T, M, N, E,
+                                      k, _stream(G.device)), "q38moe_expert_wgrad")
     return dW
 
 

@@ -396,3 +396,36 @@ def test_dropin_block_trains_under_autocast(gpu, main):
         r = _rel(got, want)
         print(f"{n}: rel L2 {r:.2e}")
         assert r <= REL, f"{n}: rel L2 {r:.3e}"
+
+
+@pytest.mark.parametrize("E,k,T,M,N,skip", [(1, 1, 4096, 512, 1024, 0),   # 8 tiles, 16 parts
+                                            (1, 1, 16384, 320, 64, 5),    # 2 tiles, 64 parts, rows left out
+                                            (1, 1, 545, 64, 192, 1),      # 2 parts of 9 and 8 slices, the last partial
+                                            (2, 2, 2049, 128, 128, 3)])   # uneven experts
+def test_expert_wgrad_split_rows(gpu, E, k, T, M, N, skip):
+    """Tiles whose rows are split over several blocks: against exact products at the same bar as
+    test_expert_wgrad, gathered and sorted, and dropped pairs contribute nothing."""
+    import ctypes
+
+    from q38.hip import ops
+    n = ctypes.c_size_t()
+    assert ops.lib.q38moe_expert_wgrad_workspace_bytes(T, M, N, E, k, ctypes.byref(n)) == 0
+    assert n.value >= 2 * 4 * E * M * N, "this shape must split its rows"
+    g = torch.Generator().manual_seed(T)
+    idx = (torch.rand(T, k, generator=g) < 0.8).int() * (E - 1)
+    if skip:
+        idx.view(-1)[torch.randperm(T * k, generator=g)[:skip]] = E
+    x = torch.randn(T, N, generator=g).to(torch.bfloat16)
+    xs = torch.randn(T * k, N, generator=g).to(torch.bfloat16)
+    G = torch.randn(T * k, M, generator=g).to(torch.bfloat16)
+    di = idx.to(gpu)
+    counts, starts, perm, _, _, _ = ops.permute(di, ops.histogram(di, E), E)
+    gathered = ops.expert_wgrad(G.to(gpu), x.to(gpu), starts, counts, k, perm=perm).cpu()
+    ordered = ops.expert_wgrad(G.to(gpu), xs.to(gpu), starts, counts, k).cpu()
+    c_ref, s_ref, p_ref = orc.permute_cpu(idx.numpy(), E)
+    for e in range(E):
+        s0, c = int(s_ref[e]), int(c_ref[e])
+        rows = torch.from_numpy(p_ref[s0:s0 + c].astype("int64"))
+        Gt = G[s0:s0 + c].float().T.contiguous()
+        assert_gemm_bf16_rounding(gathered[e], Gt, x[rows // k].float().T.contiguous(), what=f"gathered[{e}]")
+        assert_gemm_bf16_rounding(ordered[e], Gt, xs[s0:s0 + c].float().T.contiguous(), what=f"sorted[{e}]")
