@@ -438,6 +438,31 @@ int q38moe_expert_wgrad_ws(const void* G, const void* X, const int32_t* perm, co
 int q38moe_swiglu_backward(const void* dH, const void* GU, void* dGU, int64_t rows, int32_t I,
                            void* stream);
 
+/*
+ * Packed prefill trunk. The mHC residual stream X [T,4,h] fp32 (modeling:994-1031) with ssq[t] = sum of
+ * X[t]^2, which every writer of X leaves for the next sublayer; dtype is that of y and the parameters
+ * (Q38MOE_BF16 or Q38MOE_FP32). h a multiple of 64.
+ *   INIT: X[t][b] = y[t];  ADD: X[t][b] += y[t];  POST: X[t][i] = sum_j P[t][i][j] X[t][j] + post[t][i] y[t]
+ * (post [T,4] and P [T,4,4] fp32, POST only). In place.
+ */
+#define Q38MOE_MHC_INIT 0
+#define Q38MOE_MHC_ADD 1
+#define Q38MOE_MHC_POST 2
+int q38moe_mhc_update(int32_t mode, float* X, const void* y, const float* post, const float* P, float* ssq,
+                      int64_t T, int32_t h, int32_t dtype, void* stream);
+
+/*
+ * A sublayer's mHC coefficients and normed input: z = tanh(r (z0 . w_b^T)) with z0 [T,rank] fp32 = X . A^T
+ * and r = rsqrt(ssq / 4h + 1e-6); post [T,4] = 2 sigmoid(b_post + alphas[1] z[4..7]); P [T,4,4] = iters
+ * Sinkhorn steps on exp(b_res + alphas[2] z[8..23]); x_out [T,h] = (1 + norm_w) * RMS-normalised
+ * sum_b sigmoid(b_pre + alphas[0] z[0..3])_b X_b (eps), in dtype like the parameters. rank a multiple of
+ * 4 up to 128, h a multiple of 64 up to 2048.
+ */
+int q38moe_mhc_pre(const float* X, const float* ssq, const float* z0, const void* w_b, const void* b_pre,
+                   const void* b_post, const void* b_res, const void* alphas, const void* norm_w, void* x_out,
+                   float* post, float* P, int64_t T, int32_t h, int32_t rank, int32_t iters, float eps, int32_t dtype,
+                   void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1156,4 +1156,51 @@ int q38moe_block_forward_fp8(const void* x, const void* w_router, const void* wq
   return Q38MOE_OK;
 }
 
+int q38moe_mhc_update(int32_t mode, float* X, const void* y, const float* post, const float* P, float* ssq,
+                      int64_t T, int32_t h, int32_t dtype, void* stream) {
+  g_err[0] = 0;
+  Q38_CHECK(check_dtype(dtype));
+  Q38_CHECK(check_dim(h, "h"));
+  if (mode < Q38MOE_MHC_INIT || mode > Q38MOE_MHC_POST) return fail(Q38MOE_EINVAL, "unknown mode %d", mode);
+  if (T < 0 || T >= (int64_t)1 << 31) return fail(Q38MOE_EINVAL, "T must be in [0, 2^31)");
+  if (T == 0) return Q38MOE_OK;
+  Q38_CHECK(check_ptr(X, "X"));
+  Q38_CHECK(check_ptr(y, "y"));
+  Q38_CHECK(check_ptr(ssq, "ssq"));
+  if (mode == Q38MOE_MHC_POST) {
+    Q38_CHECK(check_ptr(post, "post"));
+    Q38_CHECK(check_ptr(P, "P"));
+  }
+  (void)hipGetLastError();
+  Q38_HIP(q38::launch_mhc_update(mode, X, y, post, P, ssq, T, h, dtype == Q38MOE_BF16,
+                                 static_cast<hipStream_t>(stream)),
+          "mhc update launch");
+  return Q38MOE_OK;
+}
+
+int q38moe_mhc_pre(const float* X, const float* ssq, const float* z0, const void* w_b, const void* b_pre,
+                   const void* b_post, const void* b_res, const void* alphas, const void* norm_w, void* x_out,
+                   float* post, float* P, int64_t T, int32_t h, int32_t rank, int32_t iters, float eps, int32_t dtype,
+                   void* stream) {
+  g_err[0] = 0;
+  Q38_CHECK(check_dtype(dtype));
+  Q38_CHECK(check_dim(h, "h"));
+  if (h > 2048) return fail(Q38MOE_EINVAL, "h must be <= 2048 (got %d)", h);
+  if (rank < 4 || rank > 128 || rank % 4 != 0) return fail(Q38MOE_EINVAL, "rank must be a multiple of 4 in [4, 128]");
+  if (iters < 0) return fail(Q38MOE_EINVAL, "iters must be >= 0");
+  if (T < 0 || T >= (int64_t)1 << 31) return fail(Q38MOE_EINVAL, "T must be in [0, 2^31)");
+  if (T == 0) return Q38MOE_OK;
+  Q38_CHECK(check_ptr(X, "X"));
+  Q38_CHECK(check_ptr(norm_w, "norm_w"));
+  Q38_CHECK(check_ptr(x_out, "x_out"));
+  if (ssq == nullptr || z0 == nullptr || w_b == nullptr || b_pre == nullptr || b_post == nullptr ||
+      b_res == nullptr || alphas == nullptr || post == nullptr || P == nullptr)
+    return fail(Q38MOE_EINVAL, "pointers must not be NULL");
+  (void)hipGetLastError();
+  Q38_HIP(q38::launch_mhc_pre(X, ssq, z0, w_b, b_pre, b_post, b_res, alphas, norm_w, x_out, post, P, T, h, rank,
+                              iters, eps, dtype == Q38MOE_BF16, static_cast<hipStream_t>(stream)),
+          "mhc pre launch");
+  return Q38MOE_OK;
+}
+
 }  // extern "C"

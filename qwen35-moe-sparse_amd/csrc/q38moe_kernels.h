@@ -174,4 +174,13 @@ hipError_t launch_combine(const uint16_t* Y, const int32_t* inv, const void* idx
 hipError_t launch_quant_rows(const uint16_t* x, uint8_t* q, float* scale, int64_t R, int C,
                              hipStream_t stream);
 
+// Packed prefill trunk (q38moe_prefill.hip); parameters, x and y in bf16 (bf16) or fp32, the residual
+// stream X [T, 4, h] and its row sums of squares ssq [T] fp32.
+hipError_t launch_mhc_update(int mode, float* X, const void* y, const float* post, const float* P, float* ssq,
+                             int64_t T, int h, bool bf16, hipStream_t stream);
+hipError_t launch_mhc_pre(const float* X, const float* ssq, const float* z0, const void* Bw, const void* b_pre,
+                          const void* b_post, const void* b_res, const void* alphas, const void* norm_w,
+                          void* x_out, float* post, float* P, int64_t T, int h, int rank, int iters, float eps,
+                          bool bf16, hipStream_t stream);
+
 }  // namespace q38

@@ -618,3 +618,51 @@ def block_forward_fp8(x, w_router, wq, w_sh_gate_proj, k, logit_bias=None, retur
     if return_router:
         return out, logits, idx, w
     return out
+
+
+# ---- packed prefill trunk (q38moe_prefill.hip) -----------------------------------------------------
+
+MHC_INIT, MHC_ADD, MHC_POST = 0, 1, 2
+
+
+def _same(t, name, dtype, shape):
+    _need(t, name, dtype=dtype)
+    if tuple(t.shape) != tuple(shape):
+        raise ValueError(f"{name} must be {tuple(shape)}, got {tuple(t.shape)}")
+    return t
+
+
+def mhc_update(mode, X, y, ssq, post=None, P=None):
+    """In-place update of the mHC stream X [T,4,h] fp32 by y [T,h] (bf16 or fp32): MHC_INIT X_b = y, MHC_ADD
+    X_b += y, MHC_POST X = P X + post y (post [T,4], P [T,4,4]); ssq [T] = sum X^2."""
+    dt = _fdt(y, "y")
+    T, h = y.shape
+    _need(y, "y", dtype=dt, ndim=2)
+    _same(X, "X", torch.float32, (T, 4, h))
+    _same(ssq, "ssq", torch.float32, (T,))
+    if mode == MHC_POST:
+        _same(post, "post", torch.float32, (T, 4))
+        _same(P, "P", torch.float32, (T, 4, 4))
+    check(lib.q38moe_mhc_update(mode, _ptr(X), _ptr(y), _ptr(post), _ptr(P), _ptr(ssq), T, h, _DTYPES[dt],
+                                _stream(X.device)), "q38moe_mhc_update")
+
+
+def mhc_pre(X, ssq, z0, w_b, b_pre, b_post, b_res, alphas, norm_w, iters, eps):
+    """mHC coefficients and normed sublayer input from X [T,4,h], ssq [T] and z0 = X . A^T [T,rank]: (x [T,h]
+    in the parameters' dtype, post [T,4], P [T,4,4])."""
+    dt = _fdt(norm_w, "norm_w")
+    T, _, h = X.shape
+    rank = z0.shape[1]
+    _same(X, "X", torch.float32, (T, 4, h))
+    _same(ssq, "ssq", torch.float32, (T,))
+    _same(z0, "z0", torch.float32, (T, rank))
+    for t, n, shape in ((w_b, "w_b", (24, rank)), (b_pre, "b_pre", (4,)), (b_post, "b_post", (4,)),
+                        (b_res, "b_res", (4, 4)), (alphas, "alphas", (3,)), (norm_w, "norm_w", (h,))):
+        _same(t, n, dt, shape)
+    x = torch.empty(T, h, dtype=dt, device=X.device)
+    coef = torch.empty(T, 20, dtype=torch.float32, device=X.device)
+    post, P = coef.view(-1)[:4 * T].view(T, 4), coef.view(-1)[4 * T:].view(T, 4, 4)
+    check(lib.q38moe_mhc_pre(_ptr(X), _ptr(ssq), _ptr(z0), _ptr(w_b), _ptr(b_pre), _ptr(b_post), _ptr(b_res),
+                             _ptr(alphas), _ptr(norm_w), _ptr(x), _ptr(post), _ptr(P), T, h, rank, iters, eps,
+                             _DTYPES[dt], _stream(X.device)), "q38moe_mhc_pre")
+    return x, post, P

@@ -541,6 +541,56 @@ def _mhc_post(X, y, state):
     return torch.matmul(P, X) + post.unsqueeze(-1) * y.float().unsqueeze(2)
 
 
+def _native_trunk(M, cfg, ids):
+    """True when the trunk's own kernels (q38.hip.ops.mhc_*) take this forward: tokens and parameters
+    plain tensors on one GPU, parameters all bf16 or all fp32 and contiguous, no gradient, tracing or
+    function transform to record, and the shapes they are built for. Otherwise the torch code runs."""
+    from torch.autograd import forward_ad
+
+    if not ids.is_cuda or type(ids) is not torch.Tensor or cfg.n_branch != 4:
+        return False
+    if cfg.hidden % 64 or cfg.hidden > 2048 or cfg.mhc_rank % 4 or cfg.mhc_rank > 128:
+        return False
+    if torch.jit.is_tracing() or torch.compiler.is_compiling() or forward_ad._current_level >= 0:
+        return False
+    if torch._C._functorch.peek_interpreter_stack() is not None:
+        return False
+    dt = M.embed_tokens.weight.dtype
+    if dt not in (torch.bfloat16, torch.float32):
+        return False
+    grad = torch.is_grad_enabled()
+    return all(p.dtype == dt and p.device == ids.device and p.is_contiguous() and not (grad and p.requires_grad)
+               and type(p) in (torch.Tensor, nn.Parameter) for p in M.parameters())
+
+
+def _mhc_in(m, norm, X, ssq, cfg, dt):
+    """The normed input of a sublayer and its mixing state, from the stream X; ssq (its row sums of
+    squares) is given where the native kernels run."""
+    if ssq is None:
+        xin, st = _mhc_pre(m, X, cfg)
+        return _zc_norm(xin, norm.weight, cfg.rms_eps).to(dt), st
+    from .hip import ops
+
+    B, S, n, h = X.shape
+    z0 = F.linear(X.view(B * S, n * h), m.A.weight.float())
+    x, post, P = ops.mhc_pre(X.view(B * S, n, h), ssq, z0, m.B.weight, m.b_pre, m.b_post, m.b_res, m.alphas,
+                             norm.weight, cfg.mhc_iters, cfg.rms_eps)
+    return x.view(B, S, h), (post, P)
+
+
+def _mhc_out(X, y, state, ssq):
+    """The stream after a sublayer's output y (in place where the native kernels run)."""
+    if ssq is None:
+        return _mhc_post(X, y, state)
+    from .hip import ops
+
+    B, S, n, h = X.shape
+    if y.dtype not in (torch.bfloat16, torch.float32):
+        y = y.float()
+    ops.mhc_update(ops.MHC_POST, X.view(B * S, n, h), y.reshape(B * S, h).contiguous(), ssq, *state)
+    return X
+
+
 _P2 = (1000003, 998244353)
 _P3 = (1000033, 998244353, 1000000007)
 _MIX = 2654435761
@@ -670,25 +720,37 @@ def trunk_forward(M, cfg, ids, moe, router=None):
     dt = M.embed_tokens.weight.dtype
     e = F.embedding(ids, M.embed_tokens.weight)
     cos, sin = rope_tables(cfg, S, dt, ids.device)
-    X = e.float().unsqueeze(2).expand(-1, -1, cfg.n_branch, -1).contiguous()
+    ssq = None
+    native = _native_trunk(M, cfg, ids)
+    if native:
+        from .hip import ops
+
+        X = torch.empty(B, S, cfg.n_branch, cfg.hidden, device=ids.device)
+        ssq = torch.empty(B * S, device=ids.device)
+        Xt = X.view(B * S, cfg.n_branch, cfg.hidden)
+        ops.mhc_update(ops.MHC_INIT, Xt, e.view(B * S, cfg.hidden), ssq)
+    else:
+        X = e.float().unsqueeze(2).expand(-1, -1, cfg.n_branch, -1).contiguous()
     for i, layer in enumerate(M.layers):
-        xin, st = _mhc_pre(M.mhc[2 * i], X, cfg)
-        x = _zc_norm(xin, layer.input_layernorm.weight, cfg.rms_eps).to(dt)
+        x, st = _mhc_in(M.mhc[2 * i], layer.input_layernorm, X, ssq, cfg, dt)
         if layer.kind == "linear_attention":
             y = _delta_net(layer.linear_attn, x, cfg)
         else:
             y = _qsa(layer.self_attn, M.indexers[str(i)], x, cos, sin, cfg)
-        X = _mhc_post(X, y, st)
-        xin, st = _mhc_pre(M.mhc[2 * i + 1], X, cfg)
-        x = _zc_norm(xin, layer.post_attention_layernorm.weight, cfg.rms_eps).to(dt)
+        X = _mhc_out(X, y, st, ssq)
+        x, st = _mhc_in(M.mhc[2 * i + 1], layer.post_attention_layernorm, X, ssq, cfg, dt)
         if router is None:
             y = moe(layer.mlp, x, False)
         else:
             y, lg = moe(layer.mlp, x, True)
             router.append(lg)
-        X = _mhc_post(X, y, st)
+        X = _mhc_out(X, y, st, ssq)
         if i == 0 and M.ngram is not None:
-            X = X + _ngram_delta(M.ngram, X.mean(2).to(dt), ids, cfg).unsqueeze(2)
+            delta = _ngram_delta(M.ngram, X.mean(2).to(dt), ids, cfg)
+            if native:
+                ops.mhc_update(ops.MHC_ADD, Xt, delta.view(B * S, cfg.hidden), ssq)
+            else:
+                X = X + delta.unsqueeze(2)
     return _zc_norm(X.sum(2)[:, :length].to(dt), M.norm.weight, cfg.rms_eps)
 
 

@@ -1,0 +1,106 @@
+"""The prefill trunk's kernels (q38moe_prefill.hip) against float64 restatements of the modules they
+replace, next to the torch code of q38.prefill in the same dtype. Both evaluate the same formulas in
+fp32 with other summation orders, so the bar is the torch code's own distance from float64: at most
+1.5 times it, plus 2e-7 (a few fp32 roundings, where torch's happen to cancel)."""
+import pytest
+import torch
+
+from q38 import prefill as P
+
+pytestmark = pytest.mark.gpu
+
+
+def _rel(a, b):
+    return float((a.double() - b).norm() / b.norm())
+
+
+def _hold(native, torch_code, exact, what):
+    e, bar = _rel(native, exact), 1.5 * _rel(torch_code, exact) + 2e-7
+    assert e <= bar, f"{what}: {e:.2e} from float64, bar {bar:.2e}"
+
+
+def _fill(m, g, dev, std):
+    for name, p in m.named_parameters():
+        p.data = torch.randn(p.shape, generator=g, device=dev) * std(name)
+    return m
+
+
+def _mhc64(m, norm, X, y, cfg):
+    """Sublayer input and the stream after output y, in float64 (modeling:994-1031)."""
+    w = {n: p.detach().double() for n, p in m.named_parameters()}
+    X, n = X.double(), 4
+    f = X.flatten(2)
+    f = f * torch.rsqrt(f.pow(2).mean(-1, keepdim=True) + 1e-6)
+    z = torch.tanh(f @ w["A.weight"].t() @ w["B.weight"].t())
+    pre = torch.sigmoid(w["b_pre"] + w["alphas"][0] * z[..., :n])
+    post = 2 * torch.sigmoid(w["b_post"] + w["alphas"][1] * z[..., n:2 * n])
+    logits = w["b_res"] + w["alphas"][2] * z[..., 2 * n:].unflatten(-1, (n, n))
+    M = torch.exp(logits - logits.amax((-2, -1), keepdim=True))
+    for _ in range(cfg.mhc_iters):
+        M = M / M.sum(-1, keepdim=True)
+        M = M / M.sum(-2, keepdim=True)
+    x = (pre[..., None] * X).sum(2)
+    x = x * torch.rsqrt(x.pow(2).mean(-1, keepdim=True) + cfg.rms_eps) * (1 + norm.weight.detach().double())
+    return x, M @ X + post[..., None] * y.double()[:, :, None]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,S,h", [(1, 1, 64),        # one token, a quarter of a wave's columns
+                                   (2, 67, 320),      # a partial block of tokens, a partial chunk of columns
+                                   (1, 64, 1024),
+                                   (3, 2731, 256)])   # 16 tokens per block, the last one partial
+def test_mhc_sublayer(gpu, dtype, B, S, h):
+    """mhc_update (every mode) and mhc_pre around one sublayer."""
+    from q38.hip import ops
+    cfg = P.PrefillConfig(hidden=max(h, 64), layers=1)
+    g = torch.Generator(device=gpu).manual_seed(S + h)
+    m = _fill(P._MHC(cfg).to(gpu), g, gpu, lambda n: {"A.weight": 0.02, "B.weight": 0.2}.get(n, 1.0)).to(dtype)
+    norm = _fill(P._Norm(h).to(gpu), g, gpu, lambda n: 0.05).to(dtype)
+    e, d, y = (torch.randn(B, S, h, generator=g, device=gpu).to(dtype) for _ in range(3))
+    noise = torch.randn(B, S, 4, h, generator=g, device=gpu)
+    T = B * S
+    ssq = torch.empty(T, device=gpu)
+    with torch.no_grad():
+        X = torch.empty(B, S, 4, h, device=gpu)
+        ops.mhc_update(ops.MHC_INIT, X.view(T, 4, h), e.view(T, h), ssq)
+        ref = e.float()[:, :, None].expand(-1, -1, 4, -1)
+        assert torch.equal(X, ref)
+        ops.mhc_update(ops.MHC_ADD, X.view(T, 4, h), d.view(T, h), ssq)
+        assert torch.equal(X, ref + d.float()[:, :, None])
+        assert torch.allclose(ssq.double(), X.double().pow(2).sum((2, 3)).view(-1), rtol=1e-6)
+        X = X + noise
+        ops.mhc_update(ops.MHC_ADD, X.view(T, 4, h), torch.zeros_like(d).view(T, h), ssq)
+        start = X.clone()
+        x, st = P._mhc_in(m, norm, X, ssq, cfg, dtype)
+        X = P._mhc_out(X, y, st, ssq)
+        xt, stt = P._mhc_in(m, norm, start, None, cfg, dtype)
+        Xt = P._mhc_out(start, y, stt, None)
+        x64, X64 = _mhc64(m, norm, start, y, cfg)
+    assert x.dtype == dtype
+    _hold(x, xt, x64, "sublayer input")
+    _hold(X, Xt, X64, "stream")
+    assert torch.allclose(ssq.double(), X.double().pow(2).sum((2, 3)).view(-1), rtol=1e-6)
+
+
+def test_trunk_choice(gpu):
+    """Which forwards take the kernels: plain bf16 or fp32 parameters on the GPU without gradients. Others
+    run the torch code, and gradients still flow through it."""
+    cfg = P.PrefillConfig(vocab=128, hidden=128, layers=1, lin_k_heads=1, lin_v_heads=2, moe_ffn=64, shared_ffn=64,
+                          ngram_rows=64, experts=8, topk=2)
+    ids = torch.arange(70, device=gpu)[None] % 128
+    model = P.build(cfg, device=gpu, dtype=torch.float32, moe_forward=lambda block, x: 0.1 * x)
+    M = model.model
+    assert P._native_trunk(M, cfg, ids) and not P._native_trunk(M, cfg, ids.cpu())
+    native = model(ids)
+    M.requires_grad_(True)
+    assert not P._native_trunk(M, cfg, ids)
+    hs = P.trunk_forward(M, cfg, ids, lambda block, x, r: 0.1 * x)
+    (hs @ M.embed_tokens.weight.t()).square().mean().backward()
+    assert float(M.mhc[0].A.weight.grad.norm()) > 0 and float(M.layers[0].linear_attn.A_log.grad.norm()) > 0
+    with torch.no_grad():
+        assert P._native_trunk(M, cfg, ids)
+        M.requires_grad_(False)
+        M.norm.to(torch.float64)
+        assert not P._native_trunk(M, cfg, ids)
+        M.norm.to(torch.float32)
+    assert _rel(native, (hs @ M.embed_tokens.weight.t()).detach().double()) < 1e-5
