@@ -463,6 +463,21 @@ int q38moe_mhc_pre(const float* X, const float* ssq, const float* z0, const void
                    float* post, float* P, int64_t T, int32_t h, int32_t rank, int32_t iters, float eps, int32_t dtype,
                    void* stream);
 
+/*
+ * Gated DeltaNet (modeling:464-577) between its projections. conv: causal depthwise convolution (4 taps,
+ * conv_w [C,1,4]) and SiLU on qkv [B,S,C]. delta: gated delta rule and gated RMS norm, heads 64 wide:
+ * qkv [B,S,(2 nk + nv) 64] = the convolution's q, k, v heads (value head i reads key head i / (nv / nk)),
+ * b_lin and a_lin [B,S,nv] = the beta and decay projections, A_log and dt_bias [nv], z [B,S,nv 64],
+ * norm_w [64]; out [B,S,nv 64]. S a multiple of 64, every tensor in dtype, fp32 inside. workspace:
+ * q38moe_gdn_workspace_bytes bytes, contents arbitrary.
+ */
+int q38moe_gdn_conv(const void* qkv, const void* conv_w, void* out, int64_t B, int32_t S, int32_t C, int32_t dtype,
+                    void* stream);
+int q38moe_gdn_workspace_bytes(int64_t B, int32_t S, int32_t nk, int32_t nv, int32_t dtype, size_t* bytes);
+int q38moe_gdn_delta(const void* qkv, const void* b_lin, const void* a_lin, const void* A_log, const void* dt_bias,
+                     const void* z, const void* norm_w, void* out, int64_t B, int32_t S, int32_t nk, int32_t nv,
+                     float eps, void* workspace, size_t workspace_bytes, int32_t dtype, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1203,4 +1203,65 @@ int q38moe_mhc_pre(const float* X, const float* ssq, const float* z0, const void
   return Q38MOE_OK;
 }
 
+static int check_gdn(int64_t B, int32_t S, int32_t nk, int32_t nv) {
+  if (B < 0 || S < 0) return fail(Q38MOE_EINVAL, "B and S must be >= 0");
+  if (S % 64 != 0) return fail(Q38MOE_EINVAL, "S must be a multiple of 64 (got %d)", S);
+  if (nk < 1 || nv < nk || nv % nk != 0)
+    return fail(Q38MOE_EINVAL, "value heads must be a multiple of key heads (got %d, %d)", nk, nv);
+  if (B * (int64_t)S * (2 * nk + nv) >= (int64_t)1 << 31)
+    return fail(Q38MOE_EINVAL, "B * S * heads must be < 2^31");
+  return Q38MOE_OK;
+}
+
+int q38moe_gdn_conv(const void* qkv, const void* conv_w, void* out, int64_t B, int32_t S, int32_t C, int32_t dtype,
+                    void* stream) {
+  g_err[0] = 0;
+  Q38_CHECK(check_dtype(dtype));
+  Q38_CHECK(check_dim(C, "C"));
+  if (B < 0 || S < 0 || B * (int64_t)S >= (int64_t)1 << 31) return fail(Q38MOE_EINVAL, "bad B or S");
+  if (B == 0 || S == 0) return Q38MOE_OK;
+  if ((B * ((S + 7) / 8) * (int64_t)(C / 4) + 255) / 256 >= (int64_t)1 << 31)
+    return fail(Q38MOE_EINVAL, "B * S * C is too large");
+  Q38_CHECK(check_ptr(qkv, "qkv"));
+  Q38_CHECK(check_ptr(conv_w, "conv_w"));
+  Q38_CHECK(check_ptr(out, "out"));
+  (void)hipGetLastError();
+  Q38_HIP(q38::launch_gdn_conv(qkv, conv_w, out, B, S, C, dtype == Q38MOE_BF16, static_cast<hipStream_t>(stream)),
+          "gdn conv launch");
+  return Q38MOE_OK;
+}
+
+int q38moe_gdn_workspace_bytes(int64_t B, int32_t S, int32_t nk, int32_t nv, int32_t dtype, size_t* bytes) {
+  g_err[0] = 0;
+  Q38_CHECK(check_dtype(dtype));
+  Q38_CHECK(check_gdn(B, S, nk, nv));
+  if (bytes == nullptr) return fail(Q38MOE_EINVAL, "bytes must not be NULL");
+  *bytes = align_up(sizeof(float) * q38::gdn_workspace_floats(B, S, nv)) + elem_size(dtype) * (size_t)B * S * nv * 64;
+  return Q38MOE_OK;
+}
+
+int q38moe_gdn_delta(const void* qkv, const void* b_lin, const void* a_lin, const void* A_log, const void* dt_bias,
+                     const void* z, const void* norm_w, void* out, int64_t B, int32_t S, int32_t nk, int32_t nv,
+                     float eps, void* workspace, size_t workspace_bytes, int32_t dtype, void* stream) {
+  size_t need = 0;
+  Q38_CHECK(q38moe_gdn_workspace_bytes(B, S, nk, nv, dtype, &need));
+  if (B == 0 || S == 0) return Q38MOE_OK;
+  Q38_CHECK(check_ptr(qkv, "qkv"));
+  Q38_CHECK(check_ptr(z, "z"));
+  Q38_CHECK(check_ptr(norm_w, "norm_w"));
+  Q38_CHECK(check_ptr(out, "out"));
+  if (b_lin == nullptr || a_lin == nullptr || A_log == nullptr || dt_bias == nullptr)
+    return fail(Q38MOE_EINVAL, "b_lin, a_lin, A_log and dt_bias must not be NULL");
+  Q38_CHECK(check_ptr(workspace, "workspace"));
+  if (workspace_bytes < need)
+    return fail(Q38MOE_EWORKSPACE, "workspace holds %zu bytes, %zu needed", workspace_bytes, need);
+  float* ws = static_cast<float*>(workspace);
+  void* o_frag = static_cast<char*>(workspace) + align_up(sizeof(float) * q38::gdn_workspace_floats(B, S, nv));
+  (void)hipGetLastError();
+  Q38_HIP(q38::launch_gdn_delta(qkv, b_lin, a_lin, A_log, dt_bias, z, norm_w, ws, o_frag, out, B, S, nk, nv, eps,
+                                dtype == Q38MOE_BF16, static_cast<hipStream_t>(stream)),
+          "gated delta rule launch");
+  return Q38MOE_OK;
+}
+
 }  // extern "C"

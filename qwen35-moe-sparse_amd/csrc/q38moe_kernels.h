@@ -182,5 +182,11 @@ hipError_t launch_mhc_pre(const float* X, const float* ssq, const float* z0, con
                           const void* b_post, const void* b_res, const void* alphas, const void* norm_w,
                           void* x_out, float* post, float* P, int64_t T, int h, int rank, int iters, float eps,
                           bool bf16, hipStream_t stream);
+hipError_t launch_gdn_conv(const void* qkv, const void* w, void* out, int64_t B, int S, int C, bool bf16,
+                           hipStream_t stream);
+size_t gdn_workspace_floats(int64_t B, int S, int nv);
+hipError_t launch_gdn_delta(const void* qkv, const void* b_lin, const void* a_lin, const void* A_log,
+                            const void* dt_bias, const void* z, const void* norm_w, float* ws, void* o_frag, void* out,
+                            int64_t B, int S, int nk, int nv, float eps, bool bf16, hipStream_t stream);
 
 }  // namespace q38

@@ -1,7 +1,9 @@
-// Kernels of the packed prefill's trunk around the MoE block: the mHC residual stream
-// (modeling_qwen3_8_moe.py:994-1031). As torch operations it is a chain of passes over a large fp32
-// tensor (268 MB at 4 x 4096 tokens and hidden 1024); here each pass is one kernel. fp32 is computed in
-// fp32, and values are rounded to the parameters' dtype where the torch code rounds.
+// Kernels of the packed prefill's trunk around the MoE block: the mHC residual stream and the Gated
+// DeltaNet token mixer (modeling_qwen3_8_moe.py:994-1031, 132-349, 464-577). As torch operations both
+// are chains of passes over large fp32 tensors (the four-branch stream alone is 268 MB at 4 x 4096
+// tokens and hidden 1024) and, for the delta rule's chunk loop, some 400 launches per layer; here each
+// pass over the stream is one kernel, and the delta rule three. fp32 is computed in fp32 (MFMA forms
+// with fp32 operands), and values are rounded to the parameters' dtype where the torch code rounds.
 #include "q38moe_common.h"
 #include "q38moe_kernels.h"
 
@@ -225,6 +227,386 @@ __global__ __launch_bounds__(256) void mhc_pre_kernel(const float* __restrict__ 
   }
 }
 
+// ---- Gated DeltaNet ---------------------------------------------------------------------------
+
+// Causal depthwise convolution of 4 taps in fp32, rounded to dt, then SiLU rounded to dt
+// (modeling:184-205): qkv, out [B, S, C]. A thread owns 4 channels and GDN_TS consecutive steps (a
+// sliding window of rows in registers); products and sums are rounded one by one. HBM-bound: 105 us for
+// 273 MB at 16384 x 4160 (as torch operations on transposed fp32 copies some 1.2 ms).
+constexpr int GDN_TS = 8;
+
+template <bool BF16>
+__global__ __launch_bounds__(256) void gdn_conv_kernel(const void* __restrict__ qkv, const void* __restrict__ w,
+                                                       void* __restrict__ out, int64_t runs, int S, int C) {
+  const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int cq = C / 4;
+  const int64_t run = id / cq;  // (sequence, run of GDN_TS steps)
+  if (run >= runs) return;
+  const int c = 4 * (int)(id - run * cq);
+  const int per_seq = (S + GDN_TS - 1) / GDN_TS;
+  const int64_t b = run / per_seq;
+  const int s0 = (int)(run - b * per_seq) * GDN_TS;
+  f32x4_t taps[4];  // taps[i]: the four taps of channel c + i
+#pragma unroll
+  for (int i = 0; i < 4; ++i) taps[i] = ld4_dt<BF16>(w, 4 * (int64_t)(c + i));
+  const int64_t base = b * S * C + c;
+  f32x4_t x[3 + GDN_TS];
+#pragma unroll
+  for (int j = 0; j < 3 + GDN_TS; ++j) {
+    const int s = s0 - 3 + j;
+    x[j] = s >= 0 && s < S ? ld4_dt<BF16>(qkv, base + (int64_t)s * C) : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  }
+#pragma unroll
+  for (int j = 0; j < GDN_TS; ++j) {
+    if (s0 + j >= S) break;
+    f32x4_t y;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float a = __fmul_rn(x[j][i], taps[i][0]);
+#pragma unroll
+      for (int k = 1; k < 4; ++k) a = __fadd_rn(a, __fmul_rn(x[j + k][i], taps[i][k]));
+      y[i] = silu_f32(round_dt<BF16>(a));
+    }
+    st4_dt<BF16>(out, base + (int64_t)(s0 + j) * C, y);
+  }
+}
+
+__device__ __forceinline__ f32x4_t mfma16x16x4(float a, float b, f32x4_t c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// The gated delta rule (modeling:215-349, per token 352-413) in chunks of 64 tokens, head width 64,
+// as q38.prefill.gated_delta_rule evaluates it: with c the cumulative log-decays of a chunk,
+//   A[t, s] = beta_t e^{c_t - c_s} k_t.k_s (s < t),  (I + A) [Dv | Dk] = [beta V | beta e^c K]
+// (gdn_chunk_kernel, all chunks at once), then from chunk to chunk (gdn_scan_kernel)
+//   D = Dv - Dk S,  O = (q e^c) S + (q k^T e^{c_t - c_s})_{s <= t} D,  S <- e^{c_63} S + (k e^{c_63 - c})^T D.
+//
+// v_mfma_f32_16x16x4_f32: operand lane l holds row (or column) l % 16 at k = l / 16, result lane l rows
+// 4 (l / 16) + i of column l % 16. Products take K in the order k = 16 j + 4 (l / 16) + e, so an operand
+// is a 16-byte run per lane and j ("fragment"), and a result tile of rows 16 j .. is, register for
+// register, the right-hand fragment j of the next product. Matrices that the scan reads are kept in
+// scratch in fragment order: [.][64 lanes][4], one coalesced 16-byte access per lane.
+//
+// At 4 x 4096 tokens and 39 value heads (9984 chunks) the chunk kernel takes 320 us, the scan 290 us and
+// the norm below 62 us, where the torch operations of one layer took about 8 ms (some 400 launches; the
+// scan alone 64 x 5 small products). The chunk kernel is bound by its MFMA and LDS latency chains (two
+// workgroups per CU by LDS) and 598 MB of scratch written, the scan by its serial chain of 64 chunks x (two
+// dependent products, two barriers): 624 workgroups, 2.4 per CU.
+//
+// Fragments per chunk and head, each 64 lanes x 4 floats: Dv 16, Dk 16, K' = (k e^{c_63 - c})^T 16, the
+// lower triangle of q k^T 10; then rows' q factors and e^c.
+constexpr int GDN_C = 64;
+constexpr int GDN_FRAG = 256;  // floats per fragment
+constexpr int GDN_OFF_DK = 16 * GDN_FRAG, GDN_OFF_KW = 32 * GDN_FRAG, GDN_OFF_QK = 48 * GDN_FRAG,
+              GDN_OFF_META = 58 * GDN_FRAG;
+constexpr int GDN_CHUNK_FLOATS = GDN_OFF_META + 2 * GDN_C;
+// Tile (b, a), a <= b, of a lower triangle of 4 x 4 tiles: index b (b + 1) / 2 + a.
+__device__ __forceinline__ int tri(int b, int a) { return b * (b + 1) / 2 + a; }
+
+// One workgroup per (sequence, chunk, value head). The triangular solve is blocked by 16: the four
+// diagonal blocks are inverted by forward substitution (a column per lane), everything else is MFMA;
+// a wave owns 32 of the 128 right-hand columns, whose block solutions stay in its registers as the
+// operands of the later blocks.
+template <bool BF16>
+__global__ __launch_bounds__(256) void gdn_chunk_kernel(const void* __restrict__ qkv, const void* __restrict__ b_lin,
+                                                        const void* __restrict__ a_lin,
+                                                        const void* __restrict__ A_log,
+                                                        const void* __restrict__ dt_bias, float* __restrict__ ws,
+                                                        int S, int nk, int nv) {
+  constexpr int LD = 68;
+  __shared__ __attribute__((aligned(16))) float Ks[GDN_C * LD];
+  __shared__ __attribute__((aligned(16))) float Qs[GDN_C * LD];  // after the products: Dk, row-major
+  __shared__ __attribute__((aligned(16))) float Vs[GDN_C * LD];
+  __shared__ __attribute__((aligned(16))) float Af[10][GDN_FRAG];  // -A, fragments of tile rows
+  __shared__ __attribute__((aligned(16))) float If[4][GDN_FRAG];   // inverses of I + A's diagonal blocks
+  __shared__ float cs[GDN_C], ec[GDN_C], beta[GDN_C];
+  const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lq = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = S / GDN_C;
+  const int hv = (int)(blockIdx.x % nv), ci = (int)(blockIdx.x / nv) % n, bb = (int)(blockIdx.x / nv) / n;
+  const int hk = hv / (nv / nk);
+  const int C = (2 * nk + nv) * 64;
+  const int64_t tok0 = (int64_t)bb * S + (int64_t)ci * GDN_C;
+  float* const out = ws + ((int64_t)(bb * nv + hv) * n + ci) * GDN_CHUNK_FLOATS;
+
+  {
+    // Rows of q, k, v: thread = row tid / 4, 16 columns; q and k L2-normalised, q scaled by 64^-1/2.
+    const int row = tid >> 2, c0 = 16 * (tid & 3);
+    const int64_t at = (tok0 + row) * C;
+    f32x4_t q[4], k[4];
+    float sq = 0.0f, sk = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      q[i] = ld4_dt<BF16>(qkv, at + 64 * hk + c0 + 4 * i);
+      k[i] = ld4_dt<BF16>(qkv, at + 64 * (nk + hk) + c0 + 4 * i);
+      *reinterpret_cast<f32x4_t*>(&Vs[row * LD + c0 + 4 * i]) = ld4_dt<BF16>(qkv, at + 64 * (2 * nk + hv) + c0 + 4 * i);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        sq = fmaf(q[i][e], q[i][e], sq);
+        sk = fmaf(k[i][e], k[i][e], sk);
+      }
+    }
+    sq += __shfl_xor(sq, 1);
+    sk += __shfl_xor(sk, 1);
+    sq += __shfl_xor(sq, 2);
+    sk += __shfl_xor(sk, 2);
+    const float rq = rsqrtf(sq + 1e-6f), rk = rsqrtf(sk + 1e-6f);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      *reinterpret_cast<f32x4_t*>(&Qs[row * LD + c0 + 4 * i]) = q[i] * rq * 0.125f;
+      *reinterpret_cast<f32x4_t*>(&Ks[row * LD + c0 + 4 * i]) = k[i] * rk;
+    }
+    if ((tid & 3) == 0) out[GDN_OFF_META + row] = rq;
+  }
+  if (wave == 0) {
+    // Log-decays, their prefix sums in float64 (log-step doubling, rounded once), and beta.
+    const float x = ld_dt<BF16>(a_lin, (tok0 + lane) * nv + hv) + ld_dt<BF16>(dt_bias, hv);
+    const float sp = x > 20.0f ? x : log1pf(expf(x));
+    double c = (double)(-expf(ld_dt<BF16>(A_log, hv)) * sp);
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const double v = __shfl_up(c, o);
+      if (lane >= o) c += v;
+    }
+    cs[lane] = (float)c;
+    const float e = expf((float)c);
+    ec[lane] = e;
+    out[GDN_OFF_META + GDN_C + lane] = e;
+    beta[lane] = round_dt<BF16>(sigmoid_f32(ld_dt<BF16>(b_lin, (tok0 + lane) * nv + hv)));
+  }
+  __syncthreads();
+
+  // k_s.k_t and k_s.q_t for the tiles of the lower triangle, as products of rows s with rows t: the
+  // result lane holds column t = 16 b + l % 16, rows s = 16 a + 4 (l / 16) + i, i.e. row t's fragment.
+#pragma unroll
+  for (int u = 0; u < 5; ++u) {
+    const int pi = wave + 4 * u, pair = pi < 10 ? pi : pi - 10;
+    const int b = pair >= 6 ? 3 : pair >= 3 ? 2 : pair >= 1 ? 1 : 0, a = pair - tri(b, 0);
+    const float* rt = (pi < 10 ? Ks : Qs) + (16 * b + lr) * LD + 4 * lq;
+    const float* rs = Ks + (16 * a + lr) * LD + 4 * lq;
+    f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const f32x4_t x = *reinterpret_cast<const f32x4_t*>(rs + 16 * j);
+      const f32x4_t y = *reinterpret_cast<const f32x4_t*>(rt + 16 * j);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc = mfma16x16x4(x[e], y[e], acc);
+    }
+    const int t = 16 * b + lr;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int s = 16 * a + 4 * lq + i;
+      const float d = s <= t ? expf(cs[t] - cs[s]) : 0.0f;
+      acc[i] = pi < 10 ? (s < t ? -(beta[t] * acc[i] * d) : 0.0f) : acc[i] * d;
+    }
+    if (pi < 10) *reinterpret_cast<f32x4_t*>(&Af[pair][4 * lane]) = acc;
+    else *reinterpret_cast<f32x4_t*>(out + GDN_OFF_QK + pair * GDN_FRAG + 4 * lane) = acc;
+  }
+  __syncthreads();
+
+  {
+    // Column lr of (I + A_bb)^-1 for block b = wave: x_t = delta - sum_{s < t} A[t, s] x_s.
+    const float* blk = Af[tri(wave, wave)];
+    float x[16];
+#pragma unroll
+    for (int t = 0; t < 16; ++t) {
+      float v = t == lr ? 1.0f : 0.0f;
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        if (4 * g >= t) break;
+        const f32x4_t r = *reinterpret_cast<const f32x4_t*>(blk + 4 * (t + 16 * g));
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (4 * g + e < t) v = fmaf(r[e], x[4 * g + e], v);
+      }
+      x[t] = v;
+    }
+    if (lq == 0) {
+#pragma unroll
+      for (int t = 0; t < 16; ++t) If[wave][4 * (t + 16 * (lr >> 2)) + (lr & 3)] = x[t];
+    }
+  }
+  __syncthreads();
+
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int ct = 2 * wave + u;  // column tile: 0-3 of Dv, 4-7 of Dk
+    f32x4_t X[4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      f32x4_t acc;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int r = 16 * b + 4 * lq + i;
+        acc[i] = ct < 4 ? Vs[r * LD + 16 * ct + lr] * beta[r] : (Ks[r * LD + 16 * (ct - 4) + lr] * beta[r]) * ec[r];
+      }
+#pragma unroll
+      for (int a = 0; a < b; ++a) {
+        const f32x4_t f = *reinterpret_cast<const f32x4_t*>(&Af[tri(b, a)][4 * lane]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc = mfma16x16x4(f[e], X[a][e], acc);
+      }
+      const f32x4_t f = *reinterpret_cast<const f32x4_t*>(&If[b][4 * lane]);
+      X[b] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) X[b] = mfma16x16x4(f[e], acc[e], X[b]);
+      if (ct < 4) {
+        *reinterpret_cast<f32x4_t*>(out + (4 * b + ct) * GDN_FRAG + 4 * lane) = X[b];
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) Qs[(16 * b + 4 * lq + i) * LD + 16 * (ct - 4) + lr] = X[b][i];
+      }
+    }
+  }
+  __syncthreads();
+  const float last = cs[GDN_C - 1];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    *reinterpret_cast<f32x4_t*>(out + GDN_OFF_DK + (4 * wave + j) * GDN_FRAG + 4 * lane) =
+        *reinterpret_cast<const f32x4_t*>(&Qs[(16 * wave + lr) * LD + 16 * j + 4 * lq]);
+    f32x4_t kw;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int t = 16 * j + 4 * lq + e;
+      kw[e] = Ks[t * LD + 16 * wave + lr] * expf(last - cs[t]);
+    }
+    *reinterpret_cast<f32x4_t*>(out + GDN_OFF_KW + (4 * wave + j) * GDN_FRAG + 4 * lane) = kw;
+  }
+}
+
+// The recurrence over chunks of one (sequence, value head) and 16 of its 64 value columns (they are
+// independent): four workgroups per head, placed on one XCD (block b runs on XCD b % 8) so that the
+// fragments they share come from its L2. Wave w owns rows 16 w .. of D, O and S; the S and D fragments
+// of the others come through LDS, two barriers per chunk. Each operand register is reloaded for the
+// next chunk as soon as it is used. O goes to o_frag in dt, fragment order [chunk][w][column tile].
+template <bool BF16>
+__global__ __launch_bounds__(256, 3) void gdn_scan_kernel(const void* __restrict__ qkv, const float* __restrict__ ws,
+                                                          void* __restrict__ o_frag, int heads, int S, int nk,
+                                                          int nv) {
+  __shared__ __attribute__((aligned(16))) float Dx[4][GDN_FRAG];
+  __shared__ __attribute__((aligned(16))) float Sx[4][GDN_FRAG];
+  const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lq = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int m = (int)blockIdx.x >> 3, ct = m & 3, head = (m >> 2) * 8 + ((int)blockIdx.x & 7);
+  if (head >= heads) return;
+  const int n = S / GDN_C;
+  const int bb = head / nv, hk = (head % nv) / (nv / nk);
+  const int C = (2 * nk + nv) * 64;
+  const float* ck = ws + (int64_t)head * n * GDN_CHUNK_FLOATS;
+  const int64_t q0 = ((int64_t)bb * S + 16 * wave + lr) * C + 64 * hk + 4 * lq;
+  auto frag = [&](const float* base, int off, int i) {
+    return *reinterpret_cast<const f32x4_t*>(base + off + i * GDN_FRAG + 4 * lane);
+  };
+  f32x4_t s[4], dk[4], kw[4], qk[4], q[4], dv;
+  float rq, eq, carry;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    s[j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    dk[j] = frag(ck, GDN_OFF_DK, 4 * wave + j);
+    q[j] = ld4_dt<BF16>(qkv, q0 + 16 * j);
+    kw[j] = frag(ck, GDN_OFF_KW, 4 * wave + j);
+    qk[j] = frag(ck, GDN_OFF_QK, tri(wave, min(j, wave)));
+  }
+  dv = frag(ck, 0, 4 * wave + ct);
+  rq = ck[GDN_OFF_META + 16 * wave + lr];
+  eq = ck[GDN_OFF_META + GDN_C + 16 * wave + lr];
+  carry = load_uniform(ck + GDN_OFF_META + 2 * GDN_C - 1);
+  for (int i = 0; i < n; ++i) {
+    const float* nx = i + 1 < n ? ck + GDN_CHUNK_FLOATS : ck;
+    const int64_t qn = q0 + (int64_t)(i + 1 < n ? i + 1 : i) * GDN_C * C;
+    f32x4_t d = {0.0f, 0.0f, 0.0f, 0.0f}, o = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      f32x4_t qr;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) qr[e] = ((q[j][e] * rq) * 0.125f) * eq;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        d = mfma16x16x4(dk[j][e], s[j][e], d);
+        o = mfma16x16x4(qr[e], s[j][e], o);
+      }
+      dk[j] = frag(nx, GDN_OFF_DK, 4 * wave + j);
+      q[j] = ld4_dt<BF16>(qkv, qn + 16 * j);
+    }
+    d = dv - d;
+    *reinterpret_cast<f32x4_t*>(&Dx[wave][4 * lane]) = d;
+    dv = frag(nx, 0, 4 * wave + ct);
+    rq = nx[GDN_OFF_META + 16 * wave + lr];
+    eq = nx[GDN_OFF_META + GDN_C + 16 * wave + lr];
+    __syncthreads();
+    f32x4_t sn = s[0];  // this wave's own rows of S
+#pragma unroll
+    for (int j = 1; j < 4; ++j) sn = j == wave ? s[j] : sn;
+    sn = sn * carry;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const f32x4_t dj = *reinterpret_cast<const f32x4_t*>(&Dx[j][4 * lane]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sn = mfma16x16x4(kw[j][e], dj[e], sn);
+      if (j <= wave) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o = mfma16x16x4(qk[j][e], dj[e], o);
+      }
+    }
+    *reinterpret_cast<f32x4_t*>(&Sx[wave][4 * lane]) = sn;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      kw[j] = frag(nx, GDN_OFF_KW, 4 * wave + j);
+      qk[j] = frag(nx, GDN_OFF_QK, tri(wave, min(j, wave)));
+    }
+    carry = load_uniform(nx + GDN_OFF_META + 2 * GDN_C - 1);
+    st4_dt<BF16>(o_frag, (((int64_t)head * n + i) * 16 + 4 * wave + ct) * GDN_FRAG + 4 * lane, o);
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 4; ++j) s[j] = *reinterpret_cast<const f32x4_t*>(&Sx[j][4 * lane]);
+    ck = nx;
+  }
+}
+
+// Gated RMS norm of the heads' outputs (modeling:132-148): normalise in fp32, round to dt, times w
+// rounded, times silu(z) rounded; out [B, S, nv * 64]. One block per (chunk, head): the fragments are
+// transposed through LDS, four threads per row of 64.
+template <bool BF16>
+__global__ __launch_bounds__(256) void gdn_norm_kernel(const void* __restrict__ o_frag, const void* __restrict__ z,
+                                                       const void* __restrict__ w, void* __restrict__ out, int S,
+                                                       int nv, float eps) {
+  constexpr int LD = 68;
+  __shared__ __attribute__((aligned(16))) float os[GDN_C * LD];
+  const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lq = lane >> 4, wave = tid >> 6;
+  const int n = S / GDN_C;
+  const int hv = (int)(blockIdx.x % nv), ci = (int)(blockIdx.x / nv) % n, bb = (int)(blockIdx.x / nv) / n;
+  const int64_t chunk = (int64_t)(bb * nv + hv) * n + ci;
+#pragma unroll
+  for (int ct = 0; ct < 4; ++ct) {
+    const f32x4_t v = ld4_dt<BF16>(o_frag, (chunk * 16 + 4 * wave + ct) * GDN_FRAG + 4 * lane);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) os[(16 * wave + 4 * lq + i) * LD + 16 * ct + lr] = v[i];
+  }
+  __syncthreads();
+  const int row = tid >> 2, c0 = 16 * (tid & 3);
+  const int64_t at = ((int64_t)bb * S + ci * GDN_C + row) * nv * 64 + 64 * hv + c0;
+  f32x4_t x[4];
+  float s = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    x[i] = *reinterpret_cast<const f32x4_t*>(&os[row * LD + c0 + 4 * i]);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) s = fmaf(x[i][e], x[i][e], s);
+  }
+  s += __shfl_xor(s, 1);
+  s += __shfl_xor(s, 2);
+  const float r = rsqrtf(s / 64.0f + eps);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const f32x4_t zv = ld4_dt<BF16>(z, at + 4 * i), wv = ld4_dt<BF16>(w, c0 + 4 * i);
+    f32x4_t y;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      y[e] = round_dt<BF16>(wv[e] * round_dt<BF16>(x[i][e] * r)) * silu_f32(zv[e]);
+    st4_dt<BF16>(out, at + 4 * i, y);
+  }
+}
+
 }  // namespace
 
 hipError_t launch_mhc_update(int mode, float* X, const void* y, const float* post, const float* P, float* ssq,
@@ -283,6 +665,47 @@ hipError_t launch_mhc_pre(const float* X, const float* ssq, const float* z0, con
   }
 #undef Q38_PRE_T
   return hipGetLastError();
+}
+
+hipError_t launch_gdn_conv(const void* qkv, const void* w, void* out, int64_t B, int S, int C, bool bf16,
+                           hipStream_t stream) {
+  const int64_t runs = B * ((S + GDN_TS - 1) / GDN_TS);
+  if (runs == 0) return hipSuccess;
+  const dim3 grid((unsigned)((runs * (C / 4) + 255) / 256));
+  if (bf16) hipLaunchKernelGGL(gdn_conv_kernel<true>, grid, dim3(256), 0, stream, qkv, w, out, runs, S, C);
+  else hipLaunchKernelGGL(gdn_conv_kernel<false>, grid, dim3(256), 0, stream, qkv, w, out, runs, S, C);
+  return hipGetLastError();
+}
+
+size_t gdn_workspace_floats(int64_t B, int S, int nv) { return (size_t)B * nv * (S / GDN_C) * GDN_CHUNK_FLOATS; }
+
+template <bool BF16>
+static hipError_t launch_gdn_delta_t(const void* qkv, const void* b_lin, const void* a_lin, const void* A_log,
+                                     const void* dt_bias, const void* z, const void* norm_w, float* ws, void* o_frag,
+                                     void* out, int64_t B, int S, int nk, int nv, float eps, hipStream_t stream) {
+  const unsigned chunks = (unsigned)(B * nv * (S / GDN_C));
+  hipLaunchKernelGGL(gdn_chunk_kernel<BF16>, dim3(chunks), dim3(256), 0, stream, qkv, b_lin, a_lin, A_log, dt_bias, ws,
+                     S, nk, nv);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  const int heads = (int)(B * nv);
+  hipLaunchKernelGGL(gdn_scan_kernel<BF16>, dim3((unsigned)((heads + 7) / 8 * 32)), dim3(256), 0, stream, qkv, ws,
+                     o_frag, heads, S, nk, nv);
+  e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(gdn_norm_kernel<BF16>, dim3(chunks), dim3(256), 0, stream, o_frag, z, norm_w, out, S, nv, eps);
+  return hipGetLastError();
+}
+
+hipError_t launch_gdn_delta(const void* qkv, const void* b_lin, const void* a_lin, const void* A_log,
+                            const void* dt_bias, const void* z, const void* norm_w, float* ws, void* o_frag, void* out,
+                            int64_t B, int S, int nk, int nv, float eps, bool bf16, hipStream_t stream) {
+  if (B == 0 || S == 0) return hipSuccess;
+  if (S % GDN_C != 0 || nv % nk != 0) return hipErrorInvalidValue;
+  return bf16 ? launch_gdn_delta_t<true>(qkv, b_lin, a_lin, A_log, dt_bias, z, norm_w, ws, o_frag, out, B, S, nk, nv,
+                                         eps, stream)
+              : launch_gdn_delta_t<false>(qkv, b_lin, a_lin, A_log, dt_bias, z, norm_w, ws, o_frag, out, B, S, nk, nv,
+                                          eps, stream);
 }
 
 }  // namespace q38

@@ -666,3 +666,36 @@ def mhc_pre(X, ssq, z0, w_b, b_pre, b_post, b_res, alphas, norm_w, iters, eps):
                              _ptr(alphas), _ptr(norm_w), _ptr(x), _ptr(post), _ptr(P), T, h, rank, iters, eps,
                              _DTYPES[dt], _stream(X.device)), "q38moe_mhc_pre")
     return x, post, P
+
+
+def gdn_conv(qkv, conv_w):
+    """Causal depthwise convolution (conv_w [C,1,4]) and SiLU of qkv [B,S,C]."""
+    dt = _fdt(qkv, "qkv")
+    _need(qkv, "qkv", dtype=dt, ndim=3)
+    B, S, C = qkv.shape
+    _same(conv_w, "conv_w", dt, (C, 1, 4))
+    out = torch.empty_like(qkv)
+    check(lib.q38moe_gdn_conv(_ptr(qkv), _ptr(conv_w), _ptr(out), B, S, C, _DTYPES[dt], _stream(qkv.device)),
+          "q38moe_gdn_conv")
+    return out
+
+
+def gdn_delta(qkv, b_lin, a_lin, A_log, dt_bias, z, norm_w, nk, nv, eps):
+    """Gated delta rule and gated RMS norm of a DeltaNet layer (heads 64 wide) from the convolved qkv
+    [B,S,(2 nk + nv) 64], the projections b_lin, a_lin [B,S,nv] and z [B,S,nv 64]: [B,S,nv 64]."""
+    dt = _fdt(qkv, "qkv")
+    _need(qkv, "qkv", dtype=dt, ndim=3)
+    B, S, C = qkv.shape
+    if C != (2 * nk + nv) * 64:
+        raise ValueError(f"qkv {tuple(qkv.shape)} does not hold {nk} key and {nv} value heads of 64")
+    for t, n, shape in ((b_lin, "b_lin", (B, S, nv)), (a_lin, "a_lin", (B, S, nv)), (A_log, "A_log", (nv,)),
+                        (dt_bias, "dt_bias", (nv,)), (z, "z", (B, S, nv * 64)), (norm_w, "norm_w", (64,))):
+        _same(t, n, dt, shape)
+    n = ctypes.c_size_t()
+    check(lib.q38moe_gdn_workspace_bytes(B, S, nk, nv, _DTYPES[dt], ctypes.byref(n)), "q38moe_gdn_workspace_bytes")
+    ws = torch.empty(n.value, dtype=torch.uint8, device=qkv.device)
+    out = torch.empty_like(z)
+    check(lib.q38moe_gdn_delta(_ptr(qkv), _ptr(b_lin), _ptr(a_lin), _ptr(A_log), _ptr(dt_bias), _ptr(z), _ptr(norm_w),
+                               _ptr(out), B, S, nk, nv, eps, _ptr(ws), n.value, _DTYPES[dt], _stream(qkv.device)),
+          "q38moe_gdn_delta")
+    return out

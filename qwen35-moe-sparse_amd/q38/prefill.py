@@ -411,11 +411,19 @@ def gated_delta_rule(q, k, v, g, beta, chunk=64):
     return out.transpose(1, 2).to(out_dtype)
 
 
-def _delta_net(m, x, cfg):
-    """Qwen3_8MoeGatedDeltaNet.forward without cache (modeling:464-577)."""
+def _delta_net(m, x, cfg, native=False):
+    """Qwen3_8MoeGatedDeltaNet.forward without cache (modeling:464-577); native: the trunk's kernels run."""
     B, S, _ = x.shape
     nk, nv, d = cfg.lin_k_heads, cfg.lin_v_heads, cfg.lin_head_dim
     qkv = F.linear(x, m.in_proj_qkv.weight)
+    if (native and d == 64 and cfg.conv_kernel == 4 and nv % nk == 0 and S % BLK == 0
+            and B * S * (2 * nk + nv) < 2 ** 31):
+        from .hip import ops
+
+        o = ops.gdn_delta(ops.gdn_conv(qkv, m.conv1d.weight), F.linear(x, m.in_proj_b.weight),
+                          F.linear(x, m.in_proj_a.weight), m.A_log, m.dt_bias, F.linear(x, m.in_proj_z.weight),
+                          m.norm.weight, nk, nv, cfg.rms_eps)
+        return F.linear(o, m.out_proj.weight)
     # Causal depthwise convolution (kernel K, left zero padding) in fp32, then SiLU in x.dtype.
     w = m.conv1d.weight[:, 0, :].float()
     K = w.shape[1]
@@ -542,7 +550,7 @@ def _mhc_post(X, y, state):
 
 
 def _native_trunk(M, cfg, ids):
-    """True when the trunk's own kernels (q38.hip.ops.mhc_*) take this forward: tokens and parameters
+    """True when the trunk's own kernels (q38.hip.ops.mhc_*, gdn_*) take this forward: tokens and parameters
     plain tensors on one GPU, parameters all bf16 or all fp32 and contiguous, no gradient, tracing or
     function transform to record, and the shapes they are built for. Otherwise the torch code runs."""
     from torch.autograd import forward_ad
@@ -734,7 +742,7 @@ def trunk_forward(M, cfg, ids, moe, router=None):
     for i, layer in enumerate(M.layers):
         x, st = _mhc_in(M.mhc[2 * i], layer.input_layernorm, X, ssq, cfg, dt)
         if layer.kind == "linear_attention":
-            y = _delta_net(layer.linear_attn, x, cfg)
+            y = _delta_net(layer.linear_attn, x, cfg, native)
         else:
             y = _qsa(layer.self_attn, M.indexers[str(i)], x, cos, sin, cfg)
         X = _mhc_out(X, y, st, ssq)

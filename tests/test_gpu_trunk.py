@@ -4,6 +4,7 @@ fp32 with other summation orders, so the bar is the torch code's own distance fr
 1.5 times it, plus 2e-7 (a few fp32 roundings, where torch's happen to cancel)."""
 import pytest
 import torch
+import torch.nn.functional as F
 
 from q38 import prefill as P
 
@@ -80,6 +81,53 @@ def test_mhc_sublayer(gpu, dtype, B, S, h):
     _hold(x, xt, x64, "sublayer input")
     _hold(X, Xt, X64, "stream")
     assert torch.allclose(ssq.double(), X.double().pow(2).sum((2, 3)).view(-1), rtol=1e-6)
+
+
+def _delta64(m, x, cfg):
+    """The DeltaNet mixer in float64, token by token (modeling:352-413, 464-577)."""
+    w = {n: p.detach().double() for n, p in m.named_parameters()}
+    B, S, _ = x.shape
+    nk, nv, d = cfg.lin_k_heads, cfg.lin_v_heads, cfg.lin_head_dim
+    x = x.double()
+    qkv = (x @ w["in_proj_qkv.weight"].t()).transpose(1, 2)
+    qkv = F.silu(F.conv1d(F.pad(qkv, (3, 0)), w["conv1d.weight"], groups=qkv.shape[1]))
+    q, k, v = (t.reshape(B, -1, d, S).transpose(2, 3) for t in qkv.split([nk * d, nk * d, nv * d], 1))
+    q, k = ((t * torch.rsqrt(t.pow(2).sum(-1, keepdim=True) + 1e-6)).repeat_interleave(nv // nk, 1) for t in (q, k))
+    beta = torch.sigmoid(x @ w["in_proj_b.weight"].t()).transpose(1, 2)
+    g = (-w["A_log"].exp() * F.softplus(x @ w["in_proj_a.weight"].t() + w["dt_bias"])).transpose(1, 2)
+    state, out = x.new_zeros(B, nv, d, d), torch.empty_like(v)
+    for t in range(S):
+        state = state * g[:, :, t, None, None].exp()
+        u = beta[:, :, t, None] * (v[:, :, t] - (k[:, :, t, None] @ state)[:, :, 0])
+        state = state + k[:, :, t, :, None] * u[:, :, None]
+        out[:, :, t] = (q[:, :, t, None] * d ** -0.5 @ state)[:, :, 0]
+    o = out.transpose(1, 2)
+    o = o * torch.rsqrt(o.pow(2).mean(-1, keepdim=True) + cfg.rms_eps) * w["norm.weight"]
+    z = (x @ w["in_proj_z.weight"].t()).reshape(B, S, nv, d)
+    return (o * F.silu(z)).reshape(B, S, nv * d) @ w["out_proj.weight"].t()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,S,nk,nv,slow", [(1, 64, 1, 1, False),    # one chunk, one head
+                                            (2, 192, 2, 4, False),   # 8 heads, key heads shared by two
+                                            (3, 320, 3, 3, True),    # slow decays: states reach far back
+                                            (1, 1024, 13, 39, False)])
+def test_delta_net(gpu, dtype, B, S, nk, nv, slow):
+    """gdn_conv and gdn_delta inside the mixer; two runs agree bit for bit."""
+    cfg = P.PrefillConfig(hidden=256, layers=1, lin_k_heads=nk, lin_v_heads=nv)
+    g = torch.Generator(device=gpu).manual_seed(S + nv)
+    m = _fill(P._DeltaNet(cfg).to(gpu), g, gpu, lambda n: 0.05 if "proj" in n else 0.3)
+    m.A_log.data = torch.rand(nv, generator=g, device=gpu).mul(16).add(0.01).log() - (3.0 if slow else 0.0)
+    m.norm.weight.data += 1
+    m.dt_bias.data += 1
+    m = m.to(dtype)
+    x = torch.randn(B, S, 256, generator=g, device=gpu).to(dtype)
+    with torch.no_grad():
+        native, again = P._delta_net(m, x, cfg, True), P._delta_net(m, x, cfg, True)
+        torch_code = P._delta_net(m, x, cfg, False)
+        exact = _delta64(m, x, cfg)
+    assert native.dtype == dtype and torch.equal(native, again)
+    _hold(native, torch_code, exact, "mixer output")
 
 
 def test_trunk_choice(gpu):
