@@ -478,6 +478,20 @@ int q38moe_gdn_delta(const void* qkv, const void* b_lin, const void* a_lin, cons
                      const void* z, const void* norm_w, void* out, int64_t B, int32_t S, int32_t nk, int32_t nv,
                      float eps, void* workspace, size_t workspace_bytes, int32_t dtype, void* stream);
 
+/*
+ * QSA attention (modeling:1117-1165), heads 64 wide, every tensor in dtype. prep: zero-centred RMS norm (eps)
+ * and rotary embedding of the first rot features (cos, sin [S,rot]) of the queries in qg [B,S,H,128] (query,
+ * gate) and the keys k [B,S,KV,64]: q_out [B,S,H,64], k_out [B,S,KV,64]. attention: each 64-query block over
+ * the key blocks sel [B,S/64,kk] (the first min(block + 1, kk) entries, block ids; keys past the query are
+ * masked), fp32 scores and softmax, times sigmoid(gate): out [B,S,H,64]. S a multiple of 64, kk <= 8.
+ */
+int q38moe_qsa_prep(const void* qg, const void* k, const void* q_norm, const void* k_norm, const void* cos_t,
+                    const void* sin_t, void* q_out, void* k_out, int64_t B, int32_t S, int32_t H, int32_t KV,
+                    int32_t rot, float eps, int32_t dtype, void* stream);
+int q38moe_qsa_attention(const void* q, const void* k, const void* v, const void* qg, const int64_t* sel, void* out,
+                         int64_t B, int32_t S, int32_t H, int32_t KV, int32_t kk, float scale, int32_t dtype,
+                         void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1264,4 +1264,57 @@ int q38moe_gdn_delta(const void* qkv, const void* b_lin, const void* a_lin, cons
   return Q38MOE_OK;
 }
 
+static int check_qsa(int64_t B, int32_t S, int32_t H, int32_t KV) {
+  if (B < 0 || S < 0) return fail(Q38MOE_EINVAL, "B and S must be >= 0");
+  if (S % 64 != 0) return fail(Q38MOE_EINVAL, "S must be a multiple of 64 (got %d)", S);
+  if (KV < 1 || H < KV || H % KV != 0) return fail(Q38MOE_EINVAL, "H must be a multiple of KV (got %d, %d)", H, KV);
+  if (B * (int64_t)S * (H + KV) >= (int64_t)1 << 31 || H > 65535)
+    return fail(Q38MOE_EINVAL, "B * S * heads must be < 2^31");
+  return Q38MOE_OK;
+}
+
+int q38moe_qsa_prep(const void* qg, const void* k, const void* q_norm, const void* k_norm, const void* cos_t,
+                    const void* sin_t, void* q_out, void* k_out, int64_t B, int32_t S, int32_t H, int32_t KV,
+                    int32_t rot, float eps, int32_t dtype, void* stream) {
+  g_err[0] = 0;
+  Q38_CHECK(check_dtype(dtype));
+  Q38_CHECK(check_qsa(B, S, H, KV));
+  if (rot < 8 || rot > 64 || rot % 8 != 0) return fail(Q38MOE_EINVAL, "rot must be a multiple of 8 in [8, 64]");
+  if (B == 0 || S == 0) return Q38MOE_OK;
+  Q38_CHECK(check_ptr(qg, "qg"));
+  Q38_CHECK(check_ptr(k, "k"));
+  Q38_CHECK(check_ptr(q_norm, "q_norm"));
+  Q38_CHECK(check_ptr(k_norm, "k_norm"));
+  Q38_CHECK(check_ptr(cos_t, "cos"));
+  Q38_CHECK(check_ptr(sin_t, "sin"));
+  Q38_CHECK(check_ptr(q_out, "q_out"));
+  Q38_CHECK(check_ptr(k_out, "k_out"));
+  (void)hipGetLastError();
+  Q38_HIP(q38::launch_qsa_prep(qg, k, q_norm, k_norm, cos_t, sin_t, q_out, k_out, B * S, S, H, KV, rot, eps,
+                               dtype == Q38MOE_BF16, static_cast<hipStream_t>(stream)),
+          "qsa prep launch");
+  return Q38MOE_OK;
+}
+
+int q38moe_qsa_attention(const void* q, const void* k, const void* v, const void* qg, const int64_t* sel, void* out,
+                         int64_t B, int32_t S, int32_t H, int32_t KV, int32_t kk, float scale, int32_t dtype,
+                         void* stream) {
+  g_err[0] = 0;
+  Q38_CHECK(check_dtype(dtype));
+  Q38_CHECK(check_qsa(B, S, H, KV));
+  if (kk < 1 || kk > 8) return fail(Q38MOE_EINVAL, "kk must be in [1, 8] (got %d)", kk);
+  if (B == 0 || S == 0) return Q38MOE_OK;
+  Q38_CHECK(check_ptr(q, "q"));
+  Q38_CHECK(check_ptr(k, "k"));
+  Q38_CHECK(check_ptr(v, "v"));
+  Q38_CHECK(check_ptr(qg, "qg"));
+  if (sel == nullptr) return fail(Q38MOE_EINVAL, "sel must not be NULL");
+  Q38_CHECK(check_ptr(out, "out"));
+  (void)hipGetLastError();
+  Q38_HIP(q38::launch_qsa_attention(q, k, v, qg, sel, out, B, S, H, KV, kk, scale, dtype == Q38MOE_BF16,
+                                    static_cast<hipStream_t>(stream)),
+          "qsa attention launch");
+  return Q38MOE_OK;
+}
+
 }  // extern "C"

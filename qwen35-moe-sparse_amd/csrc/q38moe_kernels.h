@@ -188,5 +188,11 @@ size_t gdn_workspace_floats(int64_t B, int S, int nv);
 hipError_t launch_gdn_delta(const void* qkv, const void* b_lin, const void* a_lin, const void* A_log,
                             const void* dt_bias, const void* z, const void* norm_w, float* ws, void* o_frag, void* out,
                             int64_t B, int S, int nk, int nv, float eps, bool bf16, hipStream_t stream);
+hipError_t launch_qsa_prep(const void* qg, const void* k, const void* q_norm, const void* k_norm, const void* cos_t,
+                           const void* sin_t, void* q_out, void* k_out, int64_t T, int S, int H, int KV, int rot,
+                           float eps, bool bf16, hipStream_t stream);
+hipError_t launch_qsa_attention(const void* q, const void* k, const void* v, const void* qg, const int64_t* sel,
+                                void* out, int64_t B, int S, int H, int KV, int kk, float scale, bool bf16,
+                                hipStream_t stream);
 
 }  // namespace q38

@@ -1,5 +1,5 @@
 // Kernels of the packed prefill's trunk around the MoE block: the mHC residual stream and the Gated
-// DeltaNet token mixer (modeling_qwen3_8_moe.py:994-1031, 132-349, 464-577). As torch operations both
+// DeltaNet token mixer and the QSA attention (modeling_qwen3_8_moe.py:994-1031, 132-349, 464-577, 1117-1165). As torch operations both
 // are chains of passes over large fp32 tensors (the four-branch stream alone is 268 MB at 4 x 4096
 // tokens and hidden 1024) and, for the delta rule's chunk loop, some 400 launches per layer; here each
 // pass over the stream is one kernel, and the delta rule three. fp32 is computed in fp32 (MFMA forms
@@ -607,6 +607,253 @@ __global__ __launch_bounds__(256) void gdn_norm_kernel(const void* __restrict__ 
   }
 }
 
+// ---- QSA block-sparse attention -----------------------------------------------------------------
+
+// Zero-centred RMS norm of the query and key heads (64 wide) and the partial rotary embedding of their
+// first `rot` features (modeling:1117-1143, 580-623), roundings as the torch code's: the norm to dt, both
+// products of the rotation and their sum to dt. Queries come from the q projection [T, H, 128] (query,
+// gate), keys from [T, KV, 64]. Sixteen lanes per head, 4 features each; feature i's partner i +- rot / 2
+// lies in another of the lanes (rot a multiple of 8). HBM-bound: 65-69 us for 250 MB at 16384 x 40 heads
+// (a dozen torch passes before).
+template <bool BF16>
+__global__ __launch_bounds__(256) void qsa_prep_kernel(const void* __restrict__ qg, const void* __restrict__ k,
+                                                       const void* __restrict__ q_norm,
+                                                       const void* __restrict__ k_norm,
+                                                       const void* __restrict__ cos_t,
+                                                       const void* __restrict__ sin_t, void* __restrict__ q_out,
+                                                       void* __restrict__ k_out, int64_t rows, int S, int H, int KV,
+                                                       int rot, float eps) {
+  const int64_t row = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);  // (token, head): H query, KV key heads
+  const int l16 = threadIdx.x & 15, c = 4 * l16;
+  if (row >= rows) return;
+  const int64_t t = row / (H + KV);
+  const int hd = (int)(row - t * (H + KV));
+  const bool is_q = hd < H;
+  const f32x4_t x = is_q ? ld4_dt<BF16>(qg, (t * H + hd) * 128 + c) : ld4_dt<BF16>(k, (t * KV + hd - H) * 64 + c);
+  const f32x4_t w = ld4_dt<BF16>(is_q ? q_norm : k_norm, c);
+  float s = 0.0f;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) s = fmaf(x[e], x[e], s);
+#pragma unroll
+  for (int o = 1; o < 16; o <<= 1) s += __shfl_xor(s, o);
+  const float r = rsqrtf(s / 64.0f + eps);
+  f32x4_t y;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) y[e] = round_dt<BF16>((x[e] * r) * (1.0f + w[e]));
+  const int half = rot / 2;
+  const int src = (threadIdx.x & 48) + (c < half ? l16 + half / 4 : c < rot ? l16 - half / 4 : l16);
+  f32x4_t p;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) p[e] = __shfl(y[e], src);
+  if (c < rot) {
+    const int64_t at = (t % S) * rot + c;
+    const f32x4_t cs = ld4_dt<BF16>(cos_t, at), sn = ld4_dt<BF16>(sin_t, at);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float turned = c < half ? -p[e] : p[e];
+      y[e] = __fadd_rn(round_dt<BF16>(__fmul_rn(y[e], cs[e])), round_dt<BF16>(__fmul_rn(turned, sn[e])));
+    }
+  }
+  if (is_q) st4_dt<BF16>(q_out, (t * H + hd) * 64 + c, y);
+  else st4_dt<BF16>(k_out, (t * KV + hd - H) * 64 + c, y);
+}
+
+// Attention of each 64-query block over its selected 64-key blocks, times sigmoid of the gate
+// (modeling:1143-1165): scores, softmax and sums in fp32. A workgroup takes the query block of one
+// sequence and key head for `hpw` of the query heads that share it; the key and value blocks lie in LDS
+// (128 KiB for 8 blocks), and each wave runs 16 queries of one head over all of them with its scores (512
+// per query) in registers, so the softmax is one pass over exact maxima and nothing is rescaled.
+//
+// Scores are computed transposed (K rows x queries): result lane l holds 4 keys of query l % 16, which
+// is, register for register, the right-hand operand of O^T = V^T P^T.
+// bf16: K Q^T by mfma_f32_16x16x32_bf16 (exact products, fp32 sums). The fp32 probabilities enter V^T P^T
+// as three bf16 parts by truncation, whose sum is the probability exactly (8 + 8 + 8 bits), so the
+// products with the bf16 values are exact too and only the fp32 sums round, as in an fp32 product; V
+// fragments come through the transposing LDS read, in the scores' key order.
+// fp32: mfma_f32_16x16x4_f32 for both; the values take the keys' place in LDS after the scores, so a wave
+// runs one set of 16 queries (hpw = 2).
+// VALU-bound (exponentials and the three-way split, about 15 operations per score) next to 4 K MFMA
+// cycles per 16 queries: 385-400 us at 4 x 4096 tokens, 38 heads on 2, 8 blocks (the torch operations,
+// fp32 products on gathered blocks with 2.5 GB of scores in memory, about 5 ms).
+template <bool BF16>
+__global__ __launch_bounds__(512, 2) void qsa_attention_kernel(const void* __restrict__ q, const void* __restrict__ k,
+                                                               const void* __restrict__ v,
+                                                               const void* __restrict__ qg,
+                                                               const int64_t* __restrict__ sel,
+                                                               void* __restrict__ out, int S, int H, int KV, int kk,
+                                                               int hpw, float scale) {
+  constexpr int ROWB = BF16 ? 128 : 256;  // bytes per row of 64
+  constexpr int CPR = ROWB / 16;
+  __shared__ __attribute__((aligned(16))) uint8_t buf[512 * 256];
+  uint8_t* const kbuf = buf;
+  uint8_t* const vbuf = BF16 ? buf + 512 * 128 : buf;
+  const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lq = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nb = S / 64, G = H / KV;
+  const int qb = (int)blockIdx.x % nb, b = (int)blockIdx.x / nb, g = (int)blockIdx.y;
+  const int h0 = g * G + (int)blockIdx.z * hpw, hn = min(hpw, (g + 1) * G - h0);
+  const int nblk = min(qb + 1, kk);
+  const int64_t tok0 = (int64_t)b * S;
+  int kb[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j)
+    kb[j] = j < nblk ? min(max((int)load_uniform(sel + ((int64_t)b * nb + qb) * kk + j), 0), nb - 1) : 0;
+
+  auto copy_blocks = [&](const void* src, uint8_t* dst, bool values) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if (j >= nblk) break;
+#pragma unroll
+      for (int i = 0; i < CPR / 8; ++i) {
+        const int id = i * 512 + tid, r = id / CPR, pos = id % CPR;
+        const int c = pos ^ (!BF16 ? r & 15 : values ? 2 * ((r >> 1) & 3) : r & 7);
+        const uint8_t* s = static_cast<const uint8_t*>(src) + ((tok0 + 64 * kb[j] + r) * KV + g) * ROWB + 16 * c;
+        load_lds16(s, dst + j * 64 * ROWB + 16 * (i * 512 + 64 * wave));
+      }
+    }
+  };
+  copy_blocks(k, kbuf, false);
+  if (BF16) copy_blocks(v, vbuf, true);
+  wait_vmcnt0();
+  __syncthreads();
+
+  const uint32_t vbase = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t*)vbuf;
+  typedef short i16x4_t __attribute__((ext_vector_type(4)));
+  const int tasks = 4 * hn;  // (head, 16 queries)
+  for (int task = wave; BF16 ? task < tasks : task == wave; task += 8) {
+    const bool on = task < tasks;  // fp32: every wave passes the barriers
+    const int head = h0 + (on ? task >> 2 : 0), rg = task & 3;
+    const int64_t qtok = tok0 + 64 * qb + 16 * rg + lr;
+    f32x4_t sc[8][4];
+    const int64_t qat = (qtok * H + head) * 64;
+    u32x4_t qf16[2];
+    f32x4_t qf32[4];
+    if (BF16) {
+#pragma unroll
+      for (int s = 0; s < 2; ++s) qf16[s] = ld16(static_cast<const uint16_t*>(q) + qat + 32 * s + 8 * lq);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) qf32[j] = ld4_dt<false>(q, qat + 16 * j + 4 * lq);
+    }
+    float m = -__builtin_inff();
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if (j >= nblk) break;
+      // Keys past the query: key position 64 kb + 16 t + 4 lq + i > 64 qb + 16 rg + lr.
+      const int ahead = 64 * (kb[j] - qb) - 16 * rg - lr;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int r = 64 * j + 16 * t + lr;
+        f32x4_t a = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (BF16) {
+#pragma unroll
+          for (int s = 0; s < 2; ++s)
+            a = mfma16x16x32(ld16(kbuf + r * ROWB + (((4 * s + lq) ^ (r & 7)) << 4)), qf16[s], a);
+        } else {
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const f32x4_t f = *reinterpret_cast<const f32x4_t*>(kbuf + r * ROWB + (((4 * u + lq) ^ (r & 15)) << 4));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) a = mfma16x16x4(f[e], qf32[u][e], a);
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          a[i] = ahead + 16 * t + 4 * lq + i > 0 ? -__builtin_inff() : a[i] * scale;
+          m = fmaxf(m, a[i]);
+        }
+        sc[j][t] = a;
+      }
+    }
+    m = fmaxf(m, __shfl_xor(m, 16));
+    m = fmaxf(m, __shfl_xor(m, 32));
+    float sum = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if (j >= nblk) break;
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          sc[j][t][i] = expf(sc[j][t][i] - m);
+          sum += sc[j][t][i];
+        }
+    }
+    sum += __shfl_xor(sum, 16);
+    sum += __shfl_xor(sum, 32);
+    if (!BF16) {
+      __syncthreads();
+      copy_blocks(v, vbuf, true);
+      wait_vmcnt0();
+      __syncthreads();
+    }
+    f32x4_t o[4];
+#pragma unroll
+    for (int d = 0; d < 4; ++d) o[d] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if (j >= nblk) break;
+      if (BF16) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          // Probabilities of keys 32 u + {4 lq + e, 16 + 4 lq + e}: high, middle and low 8 bits.
+          u32x4_t part[3];
+#pragma unroll
+          for (int w = 0; w < 4; ++w) {
+            float x0 = sc[j][2 * u + (w >> 1)][2 * (w & 1)], x1 = sc[j][2 * u + (w >> 1)][2 * (w & 1) + 1];
+#pragma unroll
+            for (int z = 0; z < 3; ++z) {
+              const uint32_t b0 = __float_as_uint(x0), b1 = __float_as_uint(x1);
+              part[z][w] = __builtin_amdgcn_perm(b1, b0, 0x07060302u);  // high halves, x0 low
+              x0 -= __uint_as_float(b0 & 0xffff0000u);
+              x1 -= __uint_as_float(b1 & 0xffff0000u);
+            }
+          }
+          const int key = 64 * j + 32 * u + 4 * lq + (lr >> 2);  // row this lane addresses (second read: + 16)
+          const uint32_t row = vbase + key * 128;
+          const int sw = 2 * ((key >> 1) & 3);
+#pragma unroll
+          for (int d = 0; d < 4; ++d) {
+            const uint32_t at = row + ((((2 * d + ((lr & 3) >> 1)) ^ sw) << 4) | (8 * (lr & 1)));
+            typedef __attribute__((address_space(3))) i16x4_t* lds_t;
+            const uint2 x = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_t)(uintptr_t)at));
+            const uint2 y =
+                __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_t)(uintptr_t)(at + 16 * 128)));
+            const u32x4_t vf = {x.x, x.y, y.x, y.y};
+#pragma unroll
+            for (int z = 0; z < 3; ++z) o[d] = mfma16x16x32(vf, part[z], o[d]);
+          }
+        }
+      } else {
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int key = 64 * j + 16 * t + 4 * lq + e;
+#pragma unroll
+            for (int d = 0; d < 4; ++d) {
+              const float vf = *reinterpret_cast<const float*>(
+                  vbuf + key * ROWB + (((4 * d + (lr >> 2)) ^ (key & 15)) << 4) + 4 * (lr & 3));
+              o[d] = mfma16x16x4(vf, sc[j][t][e], o[d]);
+            }
+          }
+      }
+    }
+    if (!on) continue;
+    // Lane: features 16 d + 4 lq .. + 3 of query lr.
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      const int c = 16 * d + 4 * lq;
+      const f32x4_t gate = ld4_dt<BF16>(qg, (qtok * H + head) * 128 + 64 + c);
+      f32x4_t y;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        y[e] = round_dt<BF16>(o[d][e] / sum) * round_dt<BF16>(sigmoid_f32(gate[e]));
+      st4_dt<BF16>(out, qat + c, y);
+    }
+  }
+}
+
 }  // namespace
 
 hipError_t launch_mhc_update(int mode, float* X, const void* y, const float* post, const float* P, float* ssq,
@@ -706,6 +953,40 @@ hipError_t launch_gdn_delta(const void* qkv, const void* b_lin, const void* a_li
                                          eps, stream)
               : launch_gdn_delta_t<false>(qkv, b_lin, a_lin, A_log, dt_bias, z, norm_w, ws, o_frag, out, B, S, nk, nv,
                                           eps, stream);
+}
+
+hipError_t launch_qsa_prep(const void* qg, const void* k, const void* q_norm, const void* k_norm, const void* cos_t,
+                           const void* sin_t, void* q_out, void* k_out, int64_t T, int S, int H, int KV, int rot,
+                           float eps, bool bf16, hipStream_t stream) {
+  const int64_t rows = T * (H + KV);
+  if (rows == 0) return hipSuccess;
+  const dim3 grid((unsigned)((rows + 15) / 16));
+  if (bf16)
+    hipLaunchKernelGGL(qsa_prep_kernel<true>, grid, dim3(256), 0, stream, qg, k, q_norm, k_norm, cos_t, sin_t, q_out,
+                       k_out, rows, S, H, KV, rot, eps);
+  else
+    hipLaunchKernelGGL(qsa_prep_kernel<false>, grid, dim3(256), 0, stream, qg, k, q_norm, k_norm, cos_t, sin_t, q_out,
+                       k_out, rows, S, H, KV, rot, eps);
+  return hipGetLastError();
+}
+
+hipError_t launch_qsa_attention(const void* q, const void* k, const void* v, const void* qg, const int64_t* sel,
+                                void* out, int64_t B, int S, int H, int KV, int kk, float scale, bool bf16,
+                                hipStream_t stream) {
+  if (B == 0 || S == 0) return hipSuccess;
+  if (S % 64 != 0 || H % KV != 0 || kk < 1 || kk > 8) return hipErrorInvalidValue;
+  // Four heads per workgroup (two rounds of its eight waves on one copy of the blocks) where that still
+  // gives every CU a few workgroups; two heads, and always in fp32, otherwise.
+  const int G = H / KV;
+  const int hpw = bf16 && B * (S / 64) * KV * ((G + 3) / 4) >= 2 * device_cus() ? 4 : 2;
+  const dim3 grid((unsigned)(B * (S / 64)), (unsigned)KV, (unsigned)((G + hpw - 1) / hpw));
+  if (bf16)
+    hipLaunchKernelGGL(qsa_attention_kernel<true>, grid, dim3(512), 0, stream, q, k, v, qg, sel, out, S, H, KV, kk, hpw,
+                       scale);
+  else
+    hipLaunchKernelGGL(qsa_attention_kernel<false>, grid, dim3(512), 0, stream, q, k, v, qg, sel, out, S, H, KV, kk,
+                       hpw, scale);
+  return hipGetLastError();
 }
 
 }  // namespace q38

@@ -73,6 +73,9 @@ SIGNATURES = {
     "q38moe_swiglu_backward": (_c_int, [_vp, _vp, _vp, _c_i64, _c_i32, _vp]),
     "q38moe_mhc_update": (_c_int, [_c_i32] + [_vp] * 5 + [_c_i64, _c_i32, _c_i32, _vp]),
     "q38moe_mhc_pre": (_c_int, [_vp] * 12 + [_c_i64, _c_i32, _c_i32, _c_i32, ctypes.c_float, _c_i32, _vp]),
+    "q38moe_qsa_prep": (_c_int, [_vp] * 8 + [_c_i64, _c_i32, _c_i32, _c_i32, _c_i32, ctypes.c_float, _c_i32, _vp]),
+    "q38moe_qsa_attention": (_c_int, [_vp] * 6 + [_c_i64, _c_i32, _c_i32, _c_i32, _c_i32, ctypes.c_float, _c_i32,
+                                                  _vp]),
     "q38moe_gdn_conv": (_c_int, [_vp, _vp, _vp, _c_i64, _c_i32, _c_i32, _c_i32, _vp]),
     "q38moe_gdn_workspace_bytes": (_c_int, [_c_i64, _c_i32, _c_i32, _c_i32, _c_i32, ctypes.POINTER(_c_size)]),
     "q38moe_gdn_delta": (_c_int, [_vp] * 8 + [_c_i64, _c_i32, _c_i32, _c_i32, ctypes.c_float, _vp, _c_size, _c_i32,

@@ -699,3 +699,37 @@ def gdn_delta(qkv, b_lin, a_lin, A_log, dt_bias, z, norm_w, nk, nv, eps):
                                _ptr(out), B, S, nk, nv, eps, _ptr(ws), n.value, _DTYPES[dt], _stream(qkv.device)),
           "q38moe_gdn_delta")
     return out
+
+
+def qsa_prep(qg, k, q_norm, k_norm, cos, sin, eps):
+    """Normed and rotated queries [B,S,H,64] and keys [B,S,KV,64] of a QSA layer from the q projection
+    qg [B,S,H,128] (query, gate) and the k projection k [B,S,KV,64]; cos, sin [S,rot]."""
+    dt = _fdt(qg, "qg")
+    _need(qg, "qg", dtype=dt, ndim=4)
+    B, S, H, _ = qg.shape
+    KV, rot = k.shape[2], cos.shape[1]
+    for t, n, shape in ((qg, "qg", (B, S, H, 128)), (k, "k", (B, S, KV, 64)), (q_norm, "q_norm", (64,)),
+                        (k_norm, "k_norm", (64,)), (cos, "cos", (S, rot)), (sin, "sin", (S, rot))):
+        _same(t, n, dt, shape)
+    q_out = torch.empty(B, S, H, 64, dtype=dt, device=qg.device)
+    k_out = torch.empty(B, S, KV, 64, dtype=dt, device=qg.device)
+    check(lib.q38moe_qsa_prep(_ptr(qg), _ptr(k), _ptr(q_norm), _ptr(k_norm), _ptr(cos), _ptr(sin), _ptr(q_out),
+                              _ptr(k_out), B, S, H, KV, rot, eps, _DTYPES[dt], _stream(qg.device)), "q38moe_qsa_prep")
+    return q_out, k_out
+
+
+def qsa_attention(q, k, v, qg, sel, scale):
+    """Gated block-sparse attention: q [B,S,H,64], k, v [B,S,KV,64], the gate in qg [B,S,H,128], sel
+    [B,S/64,kk] int64 key-block ids (the first min(block + 1, kk) count): [B,S,H*64]."""
+    dt = _fdt(q, "q")
+    _need(q, "q", dtype=dt, ndim=4)
+    B, S, H, _ = q.shape
+    KV, kk = k.shape[2], sel.shape[-1]
+    for t, n, shape in ((q, "q", (B, S, H, 64)), (k, "k", (B, S, KV, 64)), (v, "v", (B, S, KV, 64)),
+                        (qg, "qg", (B, S, H, 128))):
+        _same(t, n, dt, shape)
+    _same(sel, "sel", torch.int64, (B, S // 64, kk))
+    out = torch.empty(B, S, H * 64, dtype=dt, device=q.device)
+    check(lib.q38moe_qsa_attention(_ptr(q), _ptr(k), _ptr(v), _ptr(qg), _ptr(sel), _ptr(out), B, S, H, KV, kk, scale,
+                                   _DTYPES[dt], _stream(q.device)), "q38moe_qsa_attention")
+    return out

@@ -463,20 +463,36 @@ def select_blocks(lp_blk, budget):
     return sel, valid
 
 
-def _qsa(m, ix, x, cos, sin, cfg):
+def _qsa(m, ix, x, cos, sin, cfg, native=False):
     """qsa_attention for inference (modeling:1117-1165, dense=False, no KL): lightning-indexer block
-    selection at block starts, then attention over the selected 64-token blocks."""
+    selection at block starts, then attention over the selected 64-token blocks. native: the trunk's
+    kernels run the norms, the rotary embedding and the attention."""
     B, S, _ = x.shape
     H, KV, hd = cfg.heads, cfg.kv_heads, cfg.head_dim
-    nb = S // BLK
     qg = F.linear(x, m.q_proj.weight).view(B, S, H, 2 * hd)
-    q, gate = qg[..., :hd], qg[..., hd:].reshape(B, S, H * hd)
-    q = _zc_norm(q, m.q_norm.weight, cfg.rms_eps).transpose(1, 2)
-    k = _zc_norm(F.linear(x, m.k_proj.weight).view(B, S, KV, hd), m.k_norm.weight, cfg.rms_eps).transpose(1, 2)
-    v = F.linear(x, m.v_proj.weight).view(B, S, KV, hd).transpose(1, 2)
-    q = _rotate(q, cos, sin)
-    k = _rotate(k, cos, sin)
+    k = F.linear(x, m.k_proj.weight).view(B, S, KV, hd)
+    v = F.linear(x, m.v_proj.weight).view(B, S, KV, hd)
+    rot = cos.shape[-1]
+    if (native and hd == 64 and H % KV == 0 and 1 <= cfg.qsa_blocks <= 8 and rot % 8 == 0 and 8 <= rot <= hd
+            and B * S * (H + KV) < 2 ** 31):
+        from .hip import ops
 
+        q, k = ops.qsa_prep(qg, k, m.q_norm.weight, m.k_norm.weight, cos, sin, cfg.rms_eps)
+        sel, _ = _qsa_select(ix, x, cos, sin, cfg)
+        return F.linear(ops.qsa_attention(q, k, v, qg, sel.contiguous(), hd ** -0.5), m.o_proj.weight)
+    q, gate = qg[..., :hd], qg[..., hd:].reshape(B, S, H * hd)
+    q = _rotate(_zc_norm(q, m.q_norm.weight, cfg.rms_eps).transpose(1, 2), cos, sin)
+    k = _rotate(_zc_norm(k, m.k_norm.weight, cfg.rms_eps).transpose(1, 2), cos, sin)
+    sel, valid = _qsa_select(ix, x, cos, sin, cfg)
+    o = block_sparse_attention(q, k, v.transpose(1, 2), sel, valid, hd ** -0.5)
+    o = o.transpose(1, 2).reshape(B, S, H * hd) * torch.sigmoid(gate)
+    return F.linear(o, m.o_proj.weight)
+
+
+def _qsa_select(ix, x, cos, sin, cfg):
+    """The lightning indexer's key blocks of each query block (modeling:1065-1114)."""
+    B, S, _ = x.shape
+    nb = S // BLK
     # Indexer (modeling:1065-1081): I[t, s] = sum_j w_j(t) relu(q_j(t).k(s)) / sqrt(d) at block starts.
     nih, dih = cfg.indexer_heads, cfg.indexer_head_dim
     iq = _rotate(F.linear(x, ix.wq.weight).view(B, S, nih, dih).transpose(1, 2), cos, sin)[:, :, ::BLK]
@@ -489,10 +505,7 @@ def _qsa(m, ix, x, cos, sin, cfg):
     score = score.masked_fill(keys[None, :] > starts[:, None], -1e9)
     lp = torch.log_softmax(score, dim=-1)
     lp_blk = torch.logsumexp(lp.view(B, nb, nb, BLK), dim=-1)
-    sel, valid = select_blocks(lp_blk, cfg.qsa_blocks)
-    o = block_sparse_attention(q, k, v, sel, valid, hd ** -0.5)
-    o = o.transpose(1, 2).reshape(B, S, H * hd) * torch.sigmoid(gate)
-    return F.linear(o, m.o_proj.weight)
+    return select_blocks(lp_blk, cfg.qsa_blocks)
 
 
 def block_sparse_attention(q, k, v, sel, valid, scale):
@@ -550,7 +563,7 @@ def _mhc_post(X, y, state):
 
 
 def _native_trunk(M, cfg, ids):
-    """True when the trunk's own kernels (q38.hip.ops.mhc_*, gdn_*) take this forward: tokens and parameters
+    """True when the trunk's own kernels (q38.hip.ops.mhc_*, gdn_*, qsa_*) take this forward: tokens and parameters
     plain tensors on one GPU, parameters all bf16 or all fp32 and contiguous, no gradient, tracing or
     function transform to record, and the shapes they are built for. Otherwise the torch code runs."""
     from torch.autograd import forward_ad
@@ -744,7 +757,7 @@ def trunk_forward(M, cfg, ids, moe, router=None):
         if layer.kind == "linear_attention":
             y = _delta_net(layer.linear_attn, x, cfg, native)
         else:
-            y = _qsa(layer.self_attn, M.indexers[str(i)], x, cos, sin, cfg)
+            y = _qsa(layer.self_attn, M.indexers[str(i)], x, cos, sin, cfg, native)
         X = _mhc_out(X, y, st, ssq)
         x, st = _mhc_in(M.mhc[2 * i + 1], layer.post_attention_layernorm, X, ssq, cfg, dt)
         if router is None:

@@ -130,6 +130,59 @@ def test_delta_net(gpu, dtype, B, S, nk, nv, slow):
     _hold(native, torch_code, exact, "mixer output")
 
 
+def _qsa64(m, sel, x, cos, sin, cfg):
+    """The QSA mixer in float64 over the given key blocks (modeling:1117-1165)."""
+    w = {n: p.detach().double() for n, p in m.named_parameters()}
+    B, S, _ = x.shape
+    H, KV, d, nb = cfg.heads, cfg.kv_heads, cfg.head_dim, S // 64
+    x, cos, sin = x.double(), cos.double(), sin.double()
+
+    def heads(name, n):
+        return (x @ w[name].t()).view(B, S, n, -1).transpose(1, 2)
+
+    def norm_rope(t, name):
+        t = t * torch.rsqrt(t.pow(2).mean(-1, keepdim=True) + cfg.rms_eps) * (1 + w[name])
+        r = cos.shape[-1]
+        turned = torch.cat([-t[..., r // 2:r], t[..., :r // 2]], -1)
+        return torch.cat([t[..., :r] * cos + turned * sin, t[..., r:]], -1)
+
+    q, gate = heads("q_proj.weight", H).split([d, d], -1)
+    q, k = norm_rope(q, "q_norm.weight"), norm_rope(heads("k_proj.weight", KV), "k_norm.weight")
+    k, v = (t.repeat_interleave(H // KV, 1) for t in (k, heads("v_proj.weight", KV)))
+    counts = torch.clamp(torch.arange(nb, device=x.device) + 1, max=sel.shape[-1])
+    chosen = torch.zeros(B, nb, nb, dtype=torch.bool, device=x.device)
+    for i in range(nb):
+        chosen[:, i].scatter_(1, sel[:, i, :int(counts[i])], True)
+    mask = chosen.repeat_interleave(64, 1).repeat_interleave(64, 2) & torch.ones(S, S, dtype=torch.bool,
+                                                                                 device=x.device).tril()
+    s = (q @ k.transpose(-1, -2) * d ** -0.5).masked_fill(~mask[:, None], float("-inf"))
+    o = (torch.softmax(s, -1) @ v) * torch.sigmoid(gate)
+    return o.transpose(1, 2).reshape(B, S, H * d) @ w["o_proj.weight"].t()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,S,H,KV,blocks,rotary,spread", [
+    (1, 64, 2, 2, 8, 0.25, 1.0),     # one block, one head per workgroup
+    (2, 320, 6, 2, 3, 0.5, 1.0),     # fewer blocks than the sequence has, an odd number of heads per key head
+    (1, 1024, 38, 2, 8, 0.25, 1.0),
+    (4, 1088, 10, 1, 8, 1.0, 6.0)])  # four heads per workgroup (bf16), a partial set of them; peaked softmax
+def test_qsa(gpu, dtype, B, S, H, KV, blocks, rotary, spread):
+    """qsa_prep and qsa_attention inside the mixer, on the key blocks the indexer selects."""
+    cfg = P.PrefillConfig(hidden=256, layers=1, heads=H, kv_heads=KV, qsa_blocks=blocks, partial_rotary=rotary)
+    g = torch.Generator(device=gpu).manual_seed(S + H)
+    m = _fill(P._Attention(cfg).to(gpu), g, gpu, lambda n: spread if "norm" in n else 0.06).to(dtype)
+    ix = _fill(P._Indexer(cfg).to(gpu), g, gpu, lambda n: 0.1).to(dtype)
+    x = torch.randn(B, S, 256, generator=g, device=gpu).to(dtype)
+    cos, sin = P.rope_tables(cfg, S, dtype, gpu)
+    with torch.no_grad():
+        native, again = P._qsa(m, ix, x, cos, sin, cfg, True), P._qsa(m, ix, x, cos, sin, cfg, True)
+        torch_code = P._qsa(m, ix, x, cos, sin, cfg)
+        sel, _ = P._qsa_select(ix, x, cos, sin, cfg)
+        exact = _qsa64(m, sel, x, cos, sin, cfg)
+    assert native.dtype == dtype and torch.equal(native, again)
+    _hold(native, torch_code, exact, "mixer output")
+
+
 def test_trunk_choice(gpu):
     """Which forwards take the kernels: plain bf16 or fp32 parameters on the GPU without gradients. Others
     run the torch code, and gradients still flow through it."""
