@@ -849,10 +849,23 @@ hipError_t launch_gate_up(const uint16_t* x, const int32_t* perm, const int4* ti
                       E, topk, false, nullptr, nullptr, nullptr, nullptr, stream);
 }
 
+// Down-form launches with rows of kb bytes run with the weights in registers (q38moe_gemm_wr.hip) from
+// 160 rows per group on average (a tile table's routed and shared rows from its size, to 256), and for
+// every dense range. Below, a run covers one or two of its 64-row tiles per 256 KiB of weights and the
+// 256 x 256 units here are as fast or faster: h = 1024, I = 256, 64 experts + shared: 92 rows per group 17.9
+// here against 18.9 us there, 138 rows 18.4 / 18.8, 184 rows 21.1 / 18.6, 276 rows 43 / 22.5, 1510 rows
+// 75 / 61; e4m3 h = 2048, I = 512: 138 rows 30.4 / 33.3, 230 rows 75 / 42, 3025 rows 281 / 220 us.
+static bool use_gemm_wr(int kb, const int4* tiles, int max_mtiles, int E) {
+  return gemm_wr_supported(kb) && (tiles == nullptr || (int64_t)(max_mtiles - E) * BM >= (int64_t)160 * (E + 1));
+}
+
 hipError_t launch_down(const uint16_t* H, const int4* tiles, const int32_t* ntiles_dev,
                        int max_mtiles, int64_t M_dense, const uint16_t* w_down,
                        const uint16_t* ws_down, uint16_t* Y, int N, int K, int E,
                        hipStream_t stream) {
+  if (use_gemm_wr(2 * K, tiles, max_mtiles, E))
+    return launch_down_wr(H, tiles, max_mtiles, M_dense, w_down, ws_down, Y, N, 2 * K, E, nullptr, nullptr, nullptr,
+                          stream);
   return down_impl(H, tiles, ntiles_dev, max_mtiles, M_dense, w_down, ws_down, Y, N, K, E, false, nullptr,
                    nullptr, nullptr, stream);
 }
@@ -876,6 +889,9 @@ hipError_t launch_down_fp8(const uint8_t* Hq, const int4* tiles, const int32_t* 
                            const uint8_t* wq_down, const float* s_down, const uint8_t* wq_sh_down,
                            const float* s_sh_down, uint16_t* Y, int N, int K, int E,
                            hipStream_t stream) {
+  if (use_gemm_wr(K, tiles, max_mtiles, E))
+    return launch_down_wr(Hq, tiles, max_mtiles, M_dense, wq_down, wq_sh_down, Y, N, K, E, a_scale, s_down, s_sh_down,
+                          stream);
   return down_impl(Hq, tiles, ntiles_dev, max_mtiles, M_dense, wq_down, wq_sh_down, Y, N, K, E, true, a_scale,
                    s_down, s_sh_down, stream);
 }
