@@ -243,6 +243,11 @@ P* at(void* base, size_t off) {
   return reinterpret_cast<P*>(static_cast<char*>(base) + off);
 }
 
+// Histogram rows of 16 tokens (route_tokens_per_row): ceil(T / 16) * E * 4 bytes, E <= 64, which the H
+// area holds (at least T rows of 64 bf16, its end rounded up to 256 bytes). The permutation has read
+// them before the first GEMM writes H.
+int32_t* narrow_hist(void* ws, const ExpertsWs& L) { return at<int32_t>(ws, L.H); }
+
 int check_rows(int64_t T, int32_t h, int32_t k) {
   if ((T * k + T) * (int64_t)h >= (int64_t)1 << 31)
     return fail(Q38MOE_EINVAL, "(T*k + T) * h must be < 2^31 (got T=%lld, h=%d)", (long long)T, h);
@@ -256,7 +261,7 @@ int run_experts(const void* x, const void* idx, bool idx64, const void* topk_w,
                 const void* sh_up, const void* sh_down, const void* shared_out,
                 const void* gate, void* out, int64_t T, int32_t h, int32_t E, int32_t k,
                 int32_t I, int64_t shared_rows, const int32_t* hist_ready, void* ws,
-                const ExpertsWs& L, hipStream_t st, bool f32 = false) {
+                const ExpertsWs& L, hipStream_t st, bool f32 = false, int hist_tokens = 64) {
   const int bm = q38::gemm_block_m();
   int32_t* hist = at<int32_t>(ws, L.hist);
   int32_t* counts = at<int32_t>(ws, L.counts);
@@ -271,7 +276,7 @@ int run_experts(const void* x, const void* idx, bool idx64, const void* topk_w,
     hist_ready = hist;
   }
   Q38_HIP(q38::launch_permute(idx, idx64, hist_ready, counts, starts, perm, inv, tiles, tile_count,
-                              bm, (int)L.max_tiles, (int)shared_rows, T, E, k, st),
+                              bm, (int)L.max_tiles, (int)shared_rows, T, E, k, st, nullptr, nullptr, hist_tokens),
           "permute launch");
   if (f32) {
     // fp32 path: the same permutation and tile table, fp32 GEMMs and combine.
@@ -384,13 +389,15 @@ int run_block(const void* x, const void* w_router, const void* w_gate_up, const 
     sh_out = sh;
   }
   // Router + shared gate logit + histogram (modeling:828, 831).
+  const int hist_tokens = q38::route_tokens_per_row(T, h);
+  if (hist_tokens != 64) hist = narrow_hist(workspace, L.ex);
   Q38_HIP(q38::launch_route(xb, static_cast<const uint16_t*>(w_router), static_cast<const uint16_t*>(w_sh_gate_proj),
                             nullptr, logit_bias, static_cast<uint16_t*>(logits), idx, w, gate, hist, T, h, E, k, st),
           "route launch");
   // Routed experts (+ the shared expert inside the same GEMMs) and the gated sum (modeling:829-833).
   return run_experts(x, idx, false, w, w_gate_up, w_down, L.fused ? w_sh_gate : nullptr,
                      L.fused ? w_sh_up : nullptr, L.fused ? w_sh_down : nullptr, sh_out, gate, out, T, h, E, k, I,
-                     L.fused ? T : 0, hist, workspace, L.ex, st);
+                     L.fused ? T : 0, hist, workspace, L.ex, st, false, hist_tokens);
 }
 
 // Static scratch of q38moe_block_forward_noalloc: one copy per GPU, held until the process ends.
@@ -478,12 +485,18 @@ int q38moe_route(const void* x, const void* w_router, const void* w_shared_gate,
             "route fp32 launch");
     return Q38MOE_OK;
   }
+  // The caller's histogram has 64 tokens per row: one row is the same either way, more rows of a
+  // narrow launch are counted from the indices.
+  const bool recount = hist != nullptr && T > 16 && q38::route_tokens_per_row(T, h) != 64;
   Q38_HIP(q38::launch_route(static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w_router),
                             static_cast<const uint16_t*>(w_shared_gate), nullptr, logit_bias,
                             static_cast<uint16_t*>(logits), topk_idx, static_cast<uint16_t*>(topk_w),
-                            static_cast<uint16_t*>(shared_gate_logit), hist, T, h, E, k,
+                            static_cast<uint16_t*>(shared_gate_logit), recount ? nullptr : hist, T, h, E, k,
                             static_cast<hipStream_t>(stream)),
           "route launch");
+  if (recount)
+    Q38_HIP(q38::launch_histogram(topk_idx, false, hist, T, E, k, static_cast<hipStream_t>(stream)),
+            "histogram launch");
   return Q38MOE_OK;
 }
 
@@ -1133,6 +1146,8 @@ int q38moe_block_forward_fp8(const void* x, const void* w_router, const void* wq
   float* sH = at<float>(workspace, F.sH);
   const uint16_t* xb = static_cast<const uint16_t*>(x);
   // Router, shared gate logit and histogram in bf16 (modeling:828, 831), then the tokens in e4m3.
+  const int hist_tokens = q38::route_tokens_per_row(T, h);
+  if (hist_tokens != 64) hist = narrow_hist(workspace, X);
   Q38_HIP(q38::launch_route(xb, static_cast<const uint16_t*>(w_router), static_cast<const uint16_t*>(w_sh_gate_proj),
                             nullptr, logit_bias, static_cast<uint16_t*>(logits), idx, w, gate, hist, T, h, E, k, st),
           "route launch");
@@ -1140,7 +1155,7 @@ int q38moe_block_forward_fp8(const void* x, const void* w_router, const void* wq
   // Permutation; each sorted row takes its token's scale (shared rows P + t: token t).
   Q38_HIP(q38::launch_permute(idx, false, hist, at<int32_t>(workspace, X.counts), at<int32_t>(workspace, X.starts),
                               perm, inv, tiles, tile_count, q38::gemm_block_m(), (int)X.max_tiles, (int)T, T, E, k, st,
-                              sx, sa),
+                              sx, sa, hist_tokens),
           "permute launch");
   Q38_HIP(gate_up_fp8_any(xq, sa, perm, tiles, tile_count, (int)X.max_tiles, T, k, T,
                           static_cast<const uint8_t*>(wq_gate_up), s_gate_up, static_cast<const uint8_t*>(wq_sh_gate),

@@ -24,6 +24,8 @@ hipError_t launch_route(const uint16_t* x, const uint16_t* wr, const uint16_t* w
                         const uint16_t* logits_in, const float* bias, uint16_t* logits_out,
                         int32_t* idx_out, uint16_t* w_out, uint16_t* gate_out, int32_t* hist,
                         int64_t T, int h, int E, int k, hipStream_t stream);
+// Tokens per histogram row that launch_route writes for bf16 x: 64, or 16 from its narrow blocks.
+int route_tokens_per_row(int64_t T, int h);
 
 // Selection from fp32 logits (the fp32 path): fp32 renormalised weights out.
 hipError_t launch_route_from_f32_logits(const float* logits, const float* bias, int32_t* idx_out, float* w_out,
@@ -54,7 +56,8 @@ hipError_t launch_permute(const void* idx, bool idx64, const int32_t* hist, int3
                           int32_t* starts, int32_t* perm, int32_t* inv, int4* tiles,
                           int32_t* tile_count, int block_m, int max_tiles, int shared_rows,
                           int64_t T, int E, int k, hipStream_t stream,
-                          const float* row_scale_in = nullptr, float* row_scale_out = nullptr);
+                          const float* row_scale_in = nullptr, float* row_scale_out = nullptr,
+                          int hist_tokens = 64);  // tokens per row of hist: 16 or 64
 
 // Rows per grouped-GEMM tile.
 int gemm_block_m();

@@ -12,7 +12,7 @@
 
 namespace q38 {
 
-constexpr int PERM_TOKENS = 64;  // tokens per histogram block (matches the router's blocks)
+constexpr int PERM_TOKENS = 64;  // most tokens per histogram row; hist_kernel's rows
 constexpr int PERM_KMAX = 8;
 
 template <typename IdxT>
@@ -36,7 +36,7 @@ __global__ __launch_bounds__(256) void hist_kernel(const IdxT* __restrict__ idx,
 template <typename IdxT>
 __global__ __launch_bounds__(256) void permute_kernel(
     const IdxT* __restrict__ idx, const int32_t* __restrict__ hist, int64_t T, int E, int k,
-    int nblk, int32_t* __restrict__ counts, int32_t* __restrict__ starts,
+    int ptok, int nblk, int32_t* __restrict__ counts, int32_t* __restrict__ starts,
     int32_t* __restrict__ perm, int32_t* __restrict__ inv, int4* __restrict__ tiles,
     int32_t* __restrict__ tile_count, int block_m, int max_tiles, int shared_rows,
     const float* __restrict__ row_scale_in, float* __restrict__ row_scale_out) {
@@ -55,8 +55,8 @@ __global__ __launch_bounds__(256) void permute_kernel(
 
   // This block's pairs p0 + i, i = 64 c + lane for chunks c = wave, wave + 4: loaded first, so that
   // their round trip overlaps the histogram scan's (they do not depend on it).
-  const int64_t t0 = (int64_t)b * PERM_TOKENS;
-  const int64_t t1 = min(t0 + PERM_TOKENS, T);
+  const int64_t t0 = (int64_t)b * ptok;
+  const int64_t t1 = min(t0 + ptok, T);
   const int np = (int)((t1 - t0) * k);
   const int64_t p0 = t0 * k;
   const int nchunk = (np + 63) / 64;
@@ -69,8 +69,8 @@ __global__ __launch_bounds__(256) void permute_kernel(
 
   // Expert totals over all blocks and the counts of the blocks before this one. Thread `tid`
   // sums column e over rows part, part + 4, ...; up to 64 independent loads are in flight per
-  // step (a wave's load is one contiguous 256-byte row), so the 256 rows of the benchmark's
-  // 16384 tokens take one round trip to L2.
+  // step (a wave's load is one contiguous 256-byte row), so 256 rows (16384 tokens by 64, 4096 by
+  // 16) take one round trip to L2.
   int tot = 0, bef = 0;
   if (e < E) {
     int bb = part;
@@ -84,20 +84,17 @@ __global__ __launch_bounds__(256) void permute_kernel(
         if (bb + 4 * u < b) bef += c[u];
       }
     }
-    for (; bb + 60 < nblk; bb += 64) {
+    // The rest, 64 rows a step: loads past the last row repeat it and count nothing (one round trip;
+    // one row at a time, the 15 rows of a part cost about 3 us).
+    for (; bb < nblk; bb += 64) {
       int c[16];
 #pragma unroll
-      for (int u = 0; u < 16; ++u) c[u] = hist[(int64_t)(bb + 4 * u) * E + e];
+      for (int u = 0; u < 16; ++u) c[u] = hist[(int64_t)min(bb + 4 * u, nblk - 1) * E + e];
 #pragma unroll
       for (int u = 0; u < 16; ++u) {
-        tot += c[u];
-        if (bb + 4 * u < b) bef += c[u];
+        if (bb + 4 * u < nblk) tot += c[u];
+        if (bb + 4 * u < b && bb + 4 * u < nblk) bef += c[u];
       }
-    }
-    for (; bb < nblk; bb += 4) {
-      const int c = hist[(int64_t)bb * E + e];
-      tot += c;
-      if (bb < b) bef += c;
     }
   }
   s_tot[part][e] = tot;
@@ -245,22 +242,22 @@ hipError_t launch_permute(const void* idx, bool idx64, const int32_t* hist, int3
                           int32_t* starts, int32_t* perm, int32_t* inv, int4* tiles,
                           int32_t* tile_count, int block_m, int max_tiles, int shared_rows,
                           int64_t T, int E, int k, hipStream_t stream, const float* row_scale_in,
-                          float* row_scale_out) {
+                          float* row_scale_out, int hist_tokens) {
   // At least one block, so T == 0 still writes zero counts and an empty tile table; with a tile
   // table at least E + 1 blocks, one per group's entries (blocks past the pairs' own only write
   // those): fewer would walk several groups each, one after another (at T <= 64, a single block
   // wrote all 65 groups' entries in about 25 us).
-  const int64_t nblk = (T + PERM_TOKENS - 1) / PERM_TOKENS;
+  const int64_t nblk = (T + hist_tokens - 1) / hist_tokens;
   int64_t g = nblk > 0 ? nblk : 1;
   if (tiles != nullptr && g < E + 1) g = E + 1;
   const unsigned grid = (unsigned)g;
   if (idx64)
     hipLaunchKernelGGL(permute_kernel<int64_t>, dim3(grid), dim3(256), 0, stream,
-                       (const int64_t*)idx, hist, T, E, k, (int)nblk, counts, starts, perm, inv,
+                       (const int64_t*)idx, hist, T, E, k, hist_tokens, (int)nblk, counts, starts, perm, inv,
                        tiles, tile_count, block_m, max_tiles, shared_rows, row_scale_in, row_scale_out);
   else
     hipLaunchKernelGGL(permute_kernel<int32_t>, dim3(grid), dim3(256), 0, stream,
-                       (const int32_t*)idx, hist, T, E, k, (int)nblk, counts, starts, perm, inv,
+                       (const int32_t*)idx, hist, T, E, k, hist_tokens, (int)nblk, counts, starts, perm, inv,
                        tiles, tile_count, block_m, max_tiles, shared_rows, row_scale_in, row_scale_out);
   return hipGetLastError();
 }

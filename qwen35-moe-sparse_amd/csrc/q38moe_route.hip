@@ -131,6 +131,19 @@ __device__ __forceinline__ float lane_f(float v, int src) {
 }
 __device__ __forceinline__ int lane_i(int v, int src) { return __builtin_amdgcn_readlane(v, src); }
 
+// Value of lane (lane ^ O) for O in {1, 2, 4}, by DPP (no LDS round trip): quad permutes for 1 and
+// 2; for 4, the half-row mirror (lane i of each 8 takes 7 - i) followed by the quad reverse (i takes
+// 3 - i within its quad), whose composition is i -> i ^ 4.
+template <int O>
+__device__ __forceinline__ int xor_lanes(int v) {
+  static_assert(O == 1 || O == 2 || O == 4, "xor_lanes: O in {1, 2, 4}");
+  if constexpr (O == 1) return __builtin_amdgcn_update_dpp(0, v, 0xb1, 0xf, 0xf, false);
+  else if constexpr (O == 2) return __builtin_amdgcn_update_dpp(0, v, 0x4e, 0xf, 0xf, false);
+  else return __builtin_amdgcn_update_dpp(0, __builtin_amdgcn_update_dpp(0, v, 0x141, 0xf, 0xf, false), 0x1b, 0xf, 0xf, false);
+}
+template <int O>
+__device__ __forceinline__ float xor_lanes_f(float v) { return __int_as_float(xor_lanes<O>(__float_as_int(v))); }
+
 // Number of set bits of m below the calling lane (v_mbcnt).
 __device__ __forceinline__ int bits_below(uint64_t m) {
   return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
@@ -353,44 +366,85 @@ __device__ void select_token(float p, bool all_nan, int lane, int E, int& out_id
   out_w = pr / torch_topk_sum<K>(v);
 }
 
-// Route one token held by the calling wave. z: selection input of expert `lane` (bf16 logit plus
-// the optional bias; lanes >= E ignored). The fp32 probabilities follow torch's CPU softmax bit
-// for bit; then select_token.
-template <int K>
-__device__ void route_token(float z, int lane, int E, int& out_idx, float& out_w, float* sv, int* si) {
+// The fp32 probability of expert `lane` for one token held by the calling wave, as torch's CPU
+// softmax computes it bit for bit. z: selection input of expert `lane` (bf16 logit plus the optional
+// bias; lanes >= E ignored). all_nan: the row's softmax is NaN everywhere (and p is NaN).
+__device__ __forceinline__ float token_probs(float z, int lane, int E, bool& all_nan) {
   const bool valid = lane < E;
   z = z + 0.0f;  // -0 -> +0 (the CPU adds the bias or a zero the same way; exp(+-0) is 1 either way)
   const bool has_nan = ballot64(valid && __builtin_isnan(z)) != 0ull;
   const float m = wave_max(valid ? z : -INFINITY);
-  const bool all_nan = has_nan || !__builtin_isfinite(m);  // softmax is NaN everywhere then
-  float p;
-  if (all_nan) {
-    p = __builtin_nanf("");
+  all_nan = has_nan || !__builtin_isfinite(m);  // softmax is NaN everywhere then
+  if (all_nan) return __builtin_nanf("");
+  const float ex = valid ? torch_cpu_expf(z - m) : 0.0f;
+  float sum;
+  if (E >= 16) {
+    // Lane l < 16 accumulates experts l, l+16, l+32, l+48 (absent ones add +0, exactly), then
+    // the 16 partial sums fold l ^ 8, l ^ 4, l ^ 2, l ^ 1.
+    float acc = ex;
+    const float e1 = __shfl(ex, (lane + 16) & 63), e2 = __shfl(ex, (lane + 32) & 63), e3 = __shfl(ex, (lane + 48) & 63);
+    acc = acc + e1;
+    acc = acc + e2;
+    acc = acc + e3;
+    acc = acc + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(acc), 0x128, 0xf, 0xf, false));  // ror 8
+    acc = acc + xor_lanes_f<4>(acc);
+    acc = acc + xor_lanes_f<2>(acc);
+    acc = acc + xor_lanes_f<1>(acc);
+    sum = lane_f(acc, 0);
   } else {
-    const float ex = valid ? torch_cpu_expf(z - m) : 0.0f;
-    float sum;
-    if (E >= 16) {
-      // Lane l < 16 accumulates experts l, l+16, l+32, l+48 (absent ones add +0, exactly), then
-      // the 16 partial sums fold l ^ 8, l ^ 4, l ^ 2, l ^ 1.
-      float acc = ex;
-      acc = acc + __shfl(ex, (lane + 16) & 63);
-      acc = acc + __shfl(ex, (lane + 32) & 63);
-      acc = acc + __shfl(ex, (lane + 48) & 63);
-      acc = acc + __shfl_xor(acc, 8);
-      acc = acc + __shfl_xor(acc, 4);
-      acc = acc + __shfl_xor(acc, 2);
-      acc = acc + __shfl_xor(acc, 1);
-      sum = lane_f(acc, 0);
-    } else {
-      sum = lane_f(ex, 0);
-      for (int e = 1; e < E; ++e) sum = sum + lane_f(ex, e);
-    }
-    p = ex * (1.0f / sum);
+    sum = lane_f(ex, 0);
+    for (int e = 1; e < E; ++e) sum = sum + lane_f(ex, e);
   }
+  return ex * (1.0f / sum);
+}
+
+// Route one token held by the calling wave: token_probs, then select_token.
+template <int K>
+__device__ void route_token(float z, int lane, int E, int& out_idx, float& out_w, float* sv, int* si) {
+  bool all_nan;
+  const float p = token_probs(z, lane, E, all_nan);
   select_token<K>(p, all_nan, lane, E, out_idx, out_w, sv, si);
 }
 
+// One token held by the calling wave, one expert per lane: k rounds of a wave-wide maximum, each
+// taking every occurrence of the largest remaining probability. The first k rounds count one
+// occurrence each exactly when the k + 1 largest values are distinct (one answer, whatever the
+// algorithm); else, and for rows with a NaN or a non-finite maximum, select_token replays libstdc++.
+template <int K>
+__device__ __forceinline__ void select_wave(float z, int lane, int E, int& out_idx, float& out_w, float* sv, int* si) {
+  bool replay;
+  const float p = token_probs(z, lane, E, replay);
+  const bool all_nan = replay;
+  float mv = 0.0f;
+  int mi = 0;
+  if (!all_nan) {
+    float lv = lane < E ? p : -INFINITY;
+    const int lim = min(K, E - 1);
+#pragma unroll 1
+    for (int r = 0; r < K; ++r) {
+      const float m = wave_max(lv);
+      const uint64_t at = ballot64(lv == m);
+      replay |= (r < lim && __popcll(at) > 1) || m == -INFINITY;  // v[r] == v[r + 1], or fewer than k experts
+      if (lane == r) {
+        mv = m;
+        mi = __ffsll((unsigned long long)at) - 1;
+      }
+      lv = lv == m ? -INFINITY : lv;
+    }
+  }
+  if (replay) {
+    select_token<K>(p, all_nan, lane, E, out_idx, out_w, sv, si);
+    return;
+  }
+  float v[K];
+#pragma unroll
+  for (int r = 0; r < K; ++r) v[r] = lane_f(mv, r);
+  out_idx = mi;
+  out_w = mv / torch_topk_sum<K>(v);
+}
+
 constexpr int ROUTE_TOKENS = 64;   // tokens per histogram row (and per block, unless TOK = 128)
+constexpr int NARROW_TOKENS = 16;  // tokens per histogram row and block of the narrow kernel
 constexpr int ROUTE_KCHUNK = 1024; // router-weight K columns staged in LDS at a time
 constexpr int ROUTE_WROWS = 65;    // 64 expert rows + the shared-expert gate row
 
@@ -402,20 +456,6 @@ constexpr int SEL_LANES = 8;  // lanes per token in the selection fast path
 // Outcomes of group_select: selected; tie (the row's probabilities are left in LDS for the
 // replay); NaN or a non-finite maximum (the replay starts from the logits).
 enum { SEL_DONE = 0, SEL_REPLAY_PROBS = 1, SEL_REPLAY_LOGITS = 2 };
-
-// Value of lane (lane ^ O) for O in {1, 2, 4}, by DPP (no LDS round trip): quad permutes for 1 and
-// 2; for 4, the half-row mirror (lane i of each 8 takes 7 - i) followed by the quad reverse (i takes
-// 3 - i within its quad), whose composition is i -> i ^ 4.
-template <int O>
-__device__ __forceinline__ int xor_lanes(int v) {
-  static_assert(O == 1 || O == 2 || O == 4, "xor_lanes: O in {1, 2, 4}");
-  if constexpr (O == 1) return __builtin_amdgcn_update_dpp(0, v, 0xb1, 0xf, 0xf, false);
-  else if constexpr (O == 2) return __builtin_amdgcn_update_dpp(0, v, 0x4e, 0xf, 0xf, false);
-  else return __builtin_amdgcn_update_dpp(0, __builtin_amdgcn_update_dpp(0, v, 0x141, 0xf, 0xf, false), 0x1b, 0xf, 0xf, false);
-}
-template <int O>
-__device__ __forceinline__ float xor_lanes_f(float v) { return __int_as_float(xor_lanes<O>(__float_as_int(v))); }
-
 
 // Per-token selection by a group of SEL_LANES lanes (lane s of the group holds experts s,
 // s + SEL_LANES, ...). The group computes the row's fp32 probabilities as torch's CPU softmax does
@@ -545,9 +585,7 @@ constexpr int ROUTE_THREADS = 1024;  // 16 waves: all multiply (K split), select
 // F32IO: the fp32 path (fp32 models): logits come in as fp32 (logits_in, computed by the fp32
 // router GEMM) and the renormalised weights leave as fp32 (no bf16 rounding, modeling:812 with
 // the fp32 logits dtype); x is unused.
-// SPLITK (T <= 16, one 64-token block; bf16, logits computed here): phase 1 is a split-K product
-// instead of the staged one, see below.
-template <int KT, bool F32IO, int TOK = ROUTE_TOKENS, bool SPLITK = false>
+template <int KT, bool F32IO, int TOK = ROUTE_TOKENS>
 __global__ __launch_bounds__(ROUTE_THREADS) void route_kernel(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ wr,
     const uint16_t* __restrict__ wsg, const void* __restrict__ logits_in,
@@ -555,7 +593,6 @@ __global__ __launch_bounds__(ROUTE_THREADS) void route_kernel(
     int32_t* __restrict__ idx_out, void* __restrict__ w_out,
     uint16_t* __restrict__ gate_out, int32_t* __restrict__ hist, int64_t T, int h, int E, int k) {
   static_assert(TOK == 64 || TOK == 128, "64 or 128 tokens per block");
-  static_assert(!SPLITK || (TOK == 64 && !F32IO), "split-K logits: one 64-token block, bf16");
   // Staged router weights (phase 1) and logits (from phase 2 on). With 128 tokens both do not fit
   // side by side: they share one LDS area, and the logits are written once every wave has finished
   // its MFMAs.
@@ -580,57 +617,7 @@ __global__ __launch_bounds__(ROUTE_THREADS) void route_kernel(
   if (tid < 64) s_bias[tid] = (bias != nullptr && tid < E) ? bias[tid] : 0.0f;
   if (tid == 0) s_nties = 0;
 
-  if constexpr (SPLITK) {
-    // At most 16 tokens (decode, short chunks): staging the 133 KB of router weights in LDS for one
-    // 16-token MFMA wave would serialise the copy and the multiply in one workgroup. Instead every
-    // wave multiplies the 16 token rows by all 64 + 1 weight rows over its eighth of K, both operands
-    // loaded from global memory straight into MFMA registers (all its loads in flight at once),
-    // and the eight partial sums are added in wave order through LDS, then rounded to bf16 as the
-    // staged product's logits are. Same products, another fp32 summation order.
-    const int kw = h / (ROUTE_THREADS / 64);  // multiple of 32 (h % 512 == 0)
-    const int64_t trow = (lane & 15) < T ? (lane & 15) : T - 1;
-    const uint16_t* const xa = x + trow * (int64_t)h + 8 * (lane >> 4);
-    const uint16_t* wrow[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int n = 16 * j + (lane & 15);
-      wrow[j] = wr + (int64_t)(n < E ? n : 0) * h + 8 * (lane >> 4);
-    }
-    const uint16_t* const grow = wsg != nullptr ? wsg + 8 * (lane >> 4) : nullptr;
-    f32x4_t acc[5];
-#pragma unroll
-    for (int j = 0; j < 5; ++j) acc[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    const int kbeg = wave_u * kw;
-#pragma unroll 4
-    for (int kk = 0; kk < kw; kk += 32) {
-      const int kq = kbeg + kk;
-      const u32x4_t a = ld16(xa + kq);
-      u32x4_t b[5];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) b[j] = ld16(wrow[j] + kq);
-      b[4] = grow != nullptr ? ld16(grow + kq) : u32x4_t{0u, 0u, 0u, 0u};
-#pragma unroll
-      for (int j = 0; j < 5; ++j) acc[j] = mfma16x16x32(a, b[j], acc[j]);
-    }
-    f32x4_t* const part = reinterpret_cast<f32x4_t*>(s_wl);  // [wave][tile][lane], 40 KB
-#pragma unroll
-    for (int j = 0; j < 5; ++j) part[(wave * 5 + j) * 64 + lane] = acc[j];
-    __syncthreads();
-    if (tid < 5 * 64) {
-      const int j = tid >> 6, l = tid & 63;
-      f32x4_t sum = part[j * 64 + l];
-      for (int w = 1; w < ROUTE_THREADS / 64; ++w) sum += part[(w * 5 + j) * 64 + l];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int tok = 4 * (l >> 4) + i, col = 16 * j + (l & 15);
-        if (j < 4) {
-          if (col < E) s_logit[tok][col] = round_bf16(sum[i]);
-        } else if ((l & 15) == 0 && wsg != nullptr) {
-          s_logit[tok][64] = round_bf16(sum[i]);
-        }
-      }
-    }
-  } else if (!F32IO && logits_in == nullptr) {
+  if (!F32IO && logits_in == nullptr) {
     const int ntile = (E + 15) >> 4;
     const bool gate_tile = wsg != nullptr;
     const int nrows_w = gate_tile ? ROUTE_WROWS : 64;
@@ -882,25 +869,196 @@ __global__ __launch_bounds__(ROUTE_THREADS) void route_kernel(
   }
 }
 
+// Few tokens: blocks of G x 16 tokens, a group of 16 being one token per wave for the selection.
+//
+// The 64-token block above is a chain of latencies, about 35000 clocks however few blocks a launch
+// has: 12000 until 133 KB of weights and 128 KB of x rows are in (rows read in MFMA layout arrive at
+// about 16 bytes per clock and CU), 5000 for the partial sums, 7000 for eight lanes per token
+// selecting, 8000 for the replay of ties. Here each wave multiplies the token rows by all 64 + 1
+// weight rows over its sixteenth of K, the weights copied in whole 128-byte pieces into an LDS area
+// of its own (no barrier; MFMA-layout loads of them took 2 us more per 1024 columns). The sixteen
+// partial sums of token w's logits are added by wave w with one expert per lane and stay there:
+// softmax, the k rounds of a wave-wide maximum and, where the k + 1 largest probabilities are not
+// distinct, the libstdc++ replay need no further exchange. What is left is the copy, one tie replay
+// (about 3 us) and the launch. Whole launch, back to back, 64-token blocks (T = 1 and 16: split K in
+// one block) -> now, in us:
+//   h = 1024: T = 1 8.9 -> 5.0, 16 11.4 -> 8.0, 61 15.3 -> 9.5, 1000 17.1 -> 10.3, 4096 17.3 -> 12.3
+//   h = 2048: T = 1 12.6 -> 6.4, 48 21.4 -> 12.4, 1000 23.0 -> 12.3, 4096 23.6 -> 13.9, 5003 23.2 -> 20.1
+constexpr int NARROW_WAVES = 16;
+constexpr int NARROW_STRIDE = 68;  // floats per token in LDS (65 used): 4 token rows apart = 16 banks
+
+template <int KT, int G>
+__global__ __launch_bounds__(NARROW_WAVES * 64) void route_narrow_kernel(
+    const uint16_t* __restrict__ x, const uint16_t* __restrict__ wr, const uint16_t* __restrict__ wsg,
+    const float* __restrict__ bias, uint16_t* __restrict__ logits_out, int32_t* __restrict__ idx_out,
+    uint16_t* __restrict__ w_out, uint16_t* __restrict__ gate_out, int32_t* __restrict__ hist, int64_t T, int h,
+    int E) {
+  // Weights of the current K chunk, one wave-private area each; then the partial sums of one group
+  // of 16 tokens at a time.
+  __shared__ __attribute__((aligned(16))) uint8_t s_w[NARROW_WAVES][64 * 128];
+  float (*const s_part)[NARROW_TOKENS][NARROW_STRIDE] =
+      reinterpret_cast<float (*)[NARROW_TOKENS][NARROW_STRIDE]>(&s_w[0][0]);
+  static_assert(sizeof(s_w) >= sizeof(float) * NARROW_WAVES * NARROW_TOKENS * NARROW_STRIDE, "partial sums");
+  __shared__ int s_hist[G][64];
+  __shared__ float s_sv[NARROW_WAVES][64];
+  __shared__ int s_si[NARROW_WAVES][64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int64_t tb = (int64_t)blockIdx.x * (NARROW_TOKENS * G);
+  if (tid < G * 64) s_hist[tid >> 6][tid & 63] = 0;
+  const float zb = bias != nullptr && lane < E ? bias[lane] : 0.0f;
+  const int kw = h / NARROW_WAVES;  // multiple of 32 (h % 512 == 0)
+  const int kbeg = wave * kw + 8 * (lane >> 4);
+  const uint16_t* xa[G];
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    const int64_t trow = tb + 16 * g + (lane & 15);
+    xa[g] = x + (trow < T ? trow : T - 1) * (int64_t)h + kbeg;
+  }
+  const uint16_t* const grow = wsg != nullptr ? wsg + kbeg : xa[0];
+  // Copies: 8 rows of 128 bytes each, lane l the 16-byte chunk of row 8 i + l / 8 that belongs in
+  // slot l % 8 (chunk c of row n is kept in slot c ^ (n & 7): a fragment's 16 rows read distinct
+  // banks).
+  const int cr = lane >> 3, cc = (lane & 7) ^ cr;
+  const uint16_t* const wbase = wr + wave * kw;
+  const uint8_t* const frag = s_w[wave] + (lane & 15) * 128;
+  const int fs = lane & 7, fq = lane >> 4;  // row & 7 of this lane's fragment rows; its K quarter
+  f32x4_t acc[G][5];
+#pragma unroll
+  for (int g = 0; g < G; ++g)
+#pragma unroll
+    for (int j = 0; j < 5; ++j) acc[g][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+  for (int k0 = 0; k0 < kw; k0 += 64) {
+    const bool two = kw - k0 >= 64;  // a last chunk of 32 columns copies chunk 0 to the slots past it
+    const int c = two ? cc : (cc < 4 ? cc : 0);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int n = 8 * i + cr;
+      load_lds16(wbase + (int64_t)(n < E ? n : 0) * h + k0 + c * 8, s_w[wave] + i * 1024);
+    }
+    const int k1 = two ? k0 + 32 : k0;
+    u32x4_t a[G][2];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      a[g][0] = ld16(xa[g] + k0);
+      a[g][1] = ld16(xa[g] + k1);
+    }
+    const u32x4_t sg[2] = {ld16(grow + k0), ld16(grow + k1)};
+    wait_vmcnt0();
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      if (s == 1 && !two) break;
+#pragma unroll
+      for (int j = 0; j < 5; ++j) {
+        const u32x4_t b = j < 4 ? *reinterpret_cast<const u32x4_t*>(frag + j * 2048 + ((4 * s + fq) ^ fs) * 16) : sg[s];
+#pragma unroll
+        for (int g = 0; g < G; ++g) acc[g][j] = mfma16x16x32(a[g][s], b, acc[g][j]);
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // fragments read before the next chunk's copies
+  }
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    __syncthreads();  // every wave has read its weights, or the group before: their area is free
+    float* const part = &s_part[wave][4 * (lane >> 4)][lane & 15];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) part[i * NARROW_STRIDE + 16 * j] = acc[g][j][i];
+      if ((lane & 15) == 0) part[i * NARROW_STRIDE + 64] = acc[g][4][i];
+    }
+    __syncthreads();
+    // Token `wave` of the group: the sums stay in registers, one expert per lane.
+    float zs = 0.0f;
+#pragma unroll
+    for (int w = 0; w < NARROW_WAVES; ++w) zs += s_part[w][wave][lane];
+    float gs = s_part[lane & 15][wave][64];  // part l in lane l < 16; each row of 16 folds to the total
+    gs += dpp_f(gs, 0xb1);
+    gs += dpp_f(gs, 0x4e);
+    gs += dpp_f(gs, 0x141);
+    gs += dpp_f(gs, 0x140);
+    // The selection of group g runs in a loop over the groups below: one copy of its code.
+    acc[g][0][0] = zs;
+    acc[g][0][1] = gs;
+  }
+  float z = acc[0][0][0], gl = acc[0][0][1];
+#pragma unroll 1
+  for (int g = 0; g < G; ++g) {
+    if constexpr (G > 1) {
+#pragma unroll
+      for (int u = 1; u < G; ++u)
+        if (g == u) {
+          z = acc[u][0][0];
+          gl = acc[u][0][1];
+        }
+    }
+    const int64_t t = tb + 16 * g + wave;
+    if (t >= T) break;
+    if (gate_out != nullptr && wsg != nullptr && lane == 0) gate_out[t] = (uint16_t)f32_to_bf16_rne(gl);
+    if (logits_out != nullptr && lane < E) logits_out[t * E + lane] = (uint16_t)f32_to_bf16_rne(z);
+    int oi;
+    float ow;
+    select_wave<KT>(round_bf16(z) + zb, lane, E, oi, ow, s_sv[wave], s_si[wave]);
+    if (lane < KT) {
+      idx_out[t * KT + lane] = oi;
+      w_out[t * KT + lane] = (uint16_t)f32_to_bf16_rne(ow);
+      atomicAdd(&s_hist[g][oi], 1);
+    }
+  }
+  if (hist == nullptr) return;
+  __syncthreads();
+  if (tid < G * 64 && (tid & 63) < E) {
+    const int64_t row = (int64_t)blockIdx.x * G + (tid >> 6);
+    if (row * NARROW_TOKENS < T) hist[row * E + (tid & 63)] = s_hist[tid >> 6][tid & 63];
+  }
+}
+
+// The narrow kernel's groups per block, 0 for the 64-token blocks: as long as one round of blocks (one
+// per CU, by their LDS) takes all tokens, with one group or, up to 8192 tokens on 256 CUs, two (h =
+// 2048: 23.2 -> 20.1 us at T = 5003, 23.9 -> 22.3 at 8192; h = 1024 the same within 0.4 us). Four
+// groups do not fit the registers (T = 16384: 42 us against 18). h % 512: whole MFMA steps per wave.
+static int narrow_groups(int64_t T, int h) {
+  if (h % 512 != 0) return 0;
+  const int64_t groups = (T + NARROW_TOKENS - 1) / NARROW_TOKENS, cus = device_cus();
+  return groups <= cus ? 1 : groups <= 2 * cus ? 2 : 0;
+}
+
+int route_tokens_per_row(int64_t T, int h) { return narrow_groups(T, h) > 0 ? NARROW_TOKENS : ROUTE_TOKENS; }
+
 hipError_t launch_route(const uint16_t* x, const uint16_t* wr, const uint16_t* wsg,
                         const uint16_t* logits_in, const float* bias, uint16_t* logits_out,
                         int32_t* idx_out, uint16_t* w_out, uint16_t* gate_out, int32_t* hist,
                         int64_t T, int h, int E, int k, hipStream_t stream) {
+  if (T == 0) return hipSuccess;
+  const int ng = logits_in == nullptr ? narrow_groups(T, h) : 0;
+  if (ng > 0) {
+    const dim3 grid((unsigned)((T + NARROW_TOKENS * ng - 1) / (NARROW_TOKENS * ng)));
+#define Q38_NARROW(KT, G)                                                                                          \
+  hipLaunchKernelGGL((route_narrow_kernel<KT, G>), grid, dim3(NARROW_WAVES * 64), 0, stream, x, wr, wsg, bias,     \
+                     logits_out, idx_out, w_out, gate_out, hist, T, h, E)
+#define Q38_ROUTE(KT)                     \
+  case KT:                                \
+    if (ng == 1) Q38_NARROW(KT, 1);       \
+    else Q38_NARROW(KT, 2);               \
+    break;
+    switch (k) {
+      Q38_ROUTE(1) Q38_ROUTE(2) Q38_ROUTE(3) Q38_ROUTE(4) Q38_ROUTE(5) Q38_ROUTE(6) Q38_ROUTE(7) Q38_ROUTE(8)
+      default: return hipErrorInvalidValue;
+    }
+#undef Q38_ROUTE
+#undef Q38_NARROW
+    return hipGetLastError();
+  }
   const int64_t nblk64 = (T + ROUTE_TOKENS - 1) / ROUTE_TOKENS;
-  if (nblk64 == 0) return hipSuccess;
   // One block per CU at a time (the staged router weights fill most of its LDS). When 64-token
   // blocks would take more than one round, 128-token blocks take half as many: each stages the
   // weights once for twice the tokens (configuration 4, T = 32768: 71 -> 54 us).
   const bool wide = nblk64 > device_cus();
   const int64_t nblk = wide ? (T + 127) / 128 : nblk64;
-  // Up to 16 tokens: the split-K logits (one workgroup either way).
-  const bool splitk = logits_in == nullptr && T <= 16 && h % 512 == 0;
 #define Q38_ROUTE(KT)                                                                                         \
   case KT:                                                                                                    \
-    if (splitk)                                                                                               \
-      hipLaunchKernelGGL((route_kernel<KT, false, 64, true>), dim3(1), dim3(ROUTE_THREADS), 0, stream, x, wr,  \
-                         wsg, logits_in, bias, logits_out, idx_out, w_out, gate_out, hist, T, h, E, k);       \
-    else if (wide)                                                                                            \
+    if (wide)                                                                                                 \
       hipLaunchKernelGGL((route_kernel<KT, false, 128>), dim3((unsigned)nblk), dim3(ROUTE_THREADS), 0, stream, \
                          x, wr, wsg, logits_in, bias, logits_out, idx_out, w_out, gate_out, hist, T, h, E, k); \
     else                                                                                                      \

@@ -193,3 +193,45 @@ def test_route_full(gpu, wl_name, T):
     if rows.any():
         assert (logits.cpu()[rows] != ref_logits[rows]).any(dim=1).all()
     print(f"{wl_name}: {int(rows.sum())} of {T} rows route differently from CPU-computed logits")
+
+
+@pytest.mark.parametrize("T,h,E,k", [
+    (1, 512, 64, 5),       # one token, a last chunk of 32 columns in every wave
+    (15, 1024, 64, 1),     # k = 1: torch's partial_sort path
+    (17, 1536, 17, 4),     # one full 64-column chunk and one of 32; a second block of one token
+    (64, 1024, 8, 8),      # E = k: every row has fewer than k + 1 experts
+    (4095, 512, 64, 8),    # last one-group block ragged
+    (4113, 1024, 64, 5),   # two groups of 16 per block on 256 CUs, the last block's second one partial
+    (4129, 1024, 40, 3),   # the last block without its second group
+    (8193, 512, 64, 5),    # past the narrow blocks
+])
+def test_route_few_tokens(gpu, T, h, E, k):
+    """Blocks of 16 tokens and their neighbours, logits from x: 0/1 activations and weights give exact
+    integer logits with ties in nearly every row, so logits, indices, weights, gate logits and the
+    histogram are all exact; one row is NaN. With and without the optional outputs."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(T)
+    x = (torch.rand(T, h, generator=g) < 0.25).to(torch.bfloat16)
+    wr = (torch.rand(E, h, generator=g) < 0.1).to(torch.bfloat16)
+    ws = (torch.rand(1, h, generator=g) < 0.1).to(torch.bfloat16)
+    x[T // 2, 0] = float("nan")
+    exact = (x.double() @ wr.double().T).to(torch.bfloat16)
+    gate_exact = (x.double() @ ws.double().reshape(-1)).to(torch.bfloat16)
+    assert float(exact.nan_to_num().max()) <= 256  # integers that bf16 holds
+    _, _, ridx, rw = orc.router(None, None, k, logits=exact)
+    logits, idx, w, gate, hist = ops.route(x.to(gpu), wr.to(gpu), k, w_shared_gate=ws.to(gpu), want_logits=True,
+                                           want_hist=True)
+    assert torch.equal(torch.nan_to_num(logits.cpu(), 1e4), torch.nan_to_num(exact, 1e4))
+    assert torch.equal(torch.nan_to_num(gate.cpu().reshape(-1), 1e4), torch.nan_to_num(gate_exact, 1e4))
+    assert torch.equal(idx.cpu().long(), ridx)
+    assert torch.equal(torch.nan_to_num(w.cpu(), 1e4), torch.nan_to_num(rw, 1e4))
+    blk = torch.arange(T).repeat_interleave(k) // 64
+    ref_hist = torch.zeros((T + 63) // 64, E, dtype=torch.int32)
+    ref_hist.index_put_((blk, ridx.flatten()), torch.tensor(1, dtype=torch.int32), accumulate=True)
+    assert torch.equal(hist.cpu(), ref_hist)
+    bias = torch.randn(E, generator=g)
+    _, idx2, w2, gate2, hist2 = ops.route(x.to(gpu), wr.to(gpu), k, logit_bias=bias.to(gpu))
+    assert gate2 is None and hist2 is None
+    _, _, ridx2, rw2 = orc.router(None, None, k, logit_bias=bias, logits=exact)
+    assert torch.equal(idx2.cpu().long(), ridx2)
+    assert torch.equal(torch.nan_to_num(w2.cpu(), 1e4), torch.nan_to_num(rw2, 1e4))
