@@ -431,6 +431,30 @@ int q38moe_expert_wgrad_ws(const void* G, const void* X, const int32_t* perm, co
                            int32_t k, void* workspace, size_t workspace_bytes, void* stream);
 
 /*
+ * The routed experts of a training step, one call per direction (bf16; the kernels of
+ * q38moe_histogram, _permute, _gate_up_save, _down and _combine forward, of q38moe_pair_dots or
+ * _gather_rows, _expert_wgrad_ws, _down_kn, _swiglu_backward and _combine with unit weights backward).
+ * `saved` carries the permutation, tile table, H, Y and [g | u] from forward to backward; `work` is the
+ * backward's scratch. q38moe_experts_train_bytes gives their sizes; `needs` is the set of gradients the
+ * backward is asked for (work only) and either size pointer may be NULL. Backward: a NULL dx, dw,
+ * d_gate_up or d_down is not computed. Buffers 16-byte aligned; contents need no initialisation.
+ */
+#define Q38MOE_NEED_X 1
+#define Q38MOE_NEED_TOPK_W 2
+#define Q38MOE_NEED_GATE_UP 4
+#define Q38MOE_NEED_DOWN 8
+int q38moe_experts_train_bytes(int64_t T, int32_t h, int32_t E, int32_t k, int32_t I, int32_t needs,
+                               size_t* saved_bytes, size_t* work_bytes);
+int q38moe_experts_train_forward(const void* x, const void* topk_idx, int32_t idx_is_int64, const void* topk_w,
+                                 const void* w_gate_up, const void* w_down, void* out, int64_t T, int32_t h, int32_t E,
+                                 int32_t k, int32_t I, void* saved, size_t saved_bytes, void* stream);
+int q38moe_experts_train_backward(const void* dout, const void* x, const void* topk_idx, int32_t idx_is_int64,
+                                  const void* topk_w, const void* w_gate_up, const void* w_down, const void* saved,
+                                  size_t saved_bytes, void* dx, void* dw, void* d_gate_up, void* d_down, int64_t T,
+                                  int32_t h, int32_t E, int32_t k, int32_t I, void* work, size_t work_bytes,
+                                  void* stream);
+
+/*
  * SwiGLU backward (act = bf16(silu(g)), h = bf16(act * u), inference.py:378):
  *   d_u = bf16(dh * act), d_g = bf16(bf16(dh * u) * sigmoid(g) * (1 + g * (1 - sigmoid(g))))
  * dH [rows,I], GU = [g | u] [rows,2I], dGU = [d_g | d_u] [rows,2I] bf16; I a multiple of 64.

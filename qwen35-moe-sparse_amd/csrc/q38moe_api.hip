@@ -816,6 +816,139 @@ int q38moe_expert_wgrad_ws(const void* G, const void* X, const int32_t* perm, co
                       stream);
 }
 
+// Scratch of q38moe_experts_train_backward for the gradients in `needs`.
+namespace {
+struct TrainWs {
+  size_t d_raw, dH, dGU, dxp, partial, partial_bytes, end;
+};
+int train_work_layout(int64_t T, int32_t h, int32_t E, int32_t k, int32_t I, int32_t needs, TrainWs* out) {
+  TrainWs w = {};
+  const size_t P = (size_t)(T * k);
+  size_t off = 0, part = 0, n = 0;
+  const bool rows = (needs & ~Q38MOE_NEED_TOPK_W) != 0, inner = (needs & (Q38MOE_NEED_X | Q38MOE_NEED_GATE_UP)) != 0;
+  w.d_raw = off; off = align_up(off + (rows ? 2 * P * h : 0));
+  w.dH = off; off = align_up(off + (inner ? 2 * P * I : 0));
+  w.dGU = off; off = align_up(off + (inner ? 4 * P * I : 0));
+  w.dxp = off; off = align_up(off + ((needs & Q38MOE_NEED_X) ? 2 * P * h : 0));
+  if (needs & Q38MOE_NEED_DOWN) {
+    Q38_CHECK(q38moe_expert_wgrad_workspace_bytes(T, h, I, E, k, &n));
+    part = n;
+  }
+  if (needs & Q38MOE_NEED_GATE_UP) {
+    Q38_CHECK(q38moe_expert_wgrad_workspace_bytes(T, 2 * I, h, E, k, &n));
+    part = n > part ? n : part;  // the two products run one after the other
+  }
+  w.partial = off;
+  w.partial_bytes = part;
+  w.end = align_up(off + part);
+  *out = w;
+  return Q38MOE_OK;
+}
+// Saved by the training forward: the experts' layout, then the gate/up pre-activations.
+size_t train_saved_bytes(int64_t T, int32_t k, int32_t I, const ExpertsWs& L) {
+  return align_up(L.end + 4 * (size_t)(T * k) * I);
+}
+int check_buffer(const void* p, size_t have, size_t need, const char* name) {
+  if (need > 0) Q38_CHECK(check_ptr(p, name));
+  if (have < need) return fail(Q38MOE_EWORKSPACE, "%s holds %zu bytes, %zu needed", name, have, need);
+  return Q38MOE_OK;
+}
+}  // namespace
+
+int q38moe_experts_train_bytes(int64_t T, int32_t h, int32_t E, int32_t k, int32_t I, int32_t needs,
+                               size_t* saved_bytes, size_t* work_bytes) {
+  g_err[0] = 0;
+  Q38_CHECK(check_routing(T, E, k));
+  Q38_CHECK(check_dim(h, "h"));
+  Q38_CHECK(check_dim(I, "I"));
+  if (saved_bytes != nullptr) *saved_bytes = train_saved_bytes(T, k, I, experts_layout(T, h, E, k, I, 0));
+  if (work_bytes != nullptr) {
+    TrainWs w;
+    Q38_CHECK(train_work_layout(T, h, E, k, I, needs, &w));
+    *work_bytes = w.end;
+  }
+  return Q38MOE_OK;
+}
+
+int q38moe_experts_train_forward(const void* x, const void* topk_idx, int32_t idx_is_int64, const void* topk_w,
+                                 const void* w_gate_up, const void* w_down, void* out, int64_t T, int32_t h, int32_t E,
+                                 int32_t k, int32_t I, void* saved, size_t saved_bytes, void* stream) {
+  g_err[0] = 0;
+  Q38_CHECK(check_routing(T, E, k));
+  Q38_CHECK(check_dim(h, "h"));
+  Q38_CHECK(check_dim(I, "I"));
+  const ExpertsWs L = experts_layout(T, h, E, k, I, 0);
+  Q38_CHECK(check_buffer(saved, saved_bytes, train_saved_bytes(T, k, I, L), "saved"));
+  int32_t* hist = at<int32_t>(saved, L.hist);
+  int32_t* perm = at<int32_t>(saved, L.perm);
+  int32_t* inv = at<int32_t>(saved, L.inv);
+  int32_t* tiles = at<int32_t>(saved, L.tiles);
+  int32_t* tile_count = at<int32_t>(saved, L.tile_count);
+  void* H = at<uint16_t>(saved, L.H);
+  void* Y = at<uint16_t>(saved, L.Y);
+  Q38_CHECK(q38moe_histogram(topk_idx, idx_is_int64, hist, T, E, k, stream));
+  Q38_CHECK(q38moe_permute(topk_idx, idx_is_int64, hist, at<int32_t>(saved, L.counts), at<int32_t>(saved, L.starts),
+                           perm, inv, tiles, tile_count, 0, T, E, k, stream));
+  Q38_CHECK(q38moe_gate_up_save(x, w_gate_up, perm, tiles, tile_count, H, at<uint16_t>(saved, L.end), T, h, E, k, I,
+                                stream));
+  Q38_CHECK(q38moe_down(H, w_down, nullptr, tiles, tile_count, 0, Y, T, h, E, k, I, Q38MOE_BF16, stream));
+  return q38moe_combine(Y, inv, topk_idx, idx_is_int64, topk_w, nullptr, nullptr, out, T, h, E, k, Q38MOE_BF16, stream);
+}
+
+int q38moe_experts_train_backward(const void* dout, const void* x, const void* topk_idx, int32_t idx_is_int64,
+                                  const void* topk_w, const void* w_gate_up, const void* w_down, const void* saved,
+                                  size_t saved_bytes, void* dx, void* dw, void* d_gate_up, void* d_down, int64_t T,
+                                  int32_t h, int32_t E, int32_t k, int32_t I, void* work, size_t work_bytes,
+                                  void* stream) {
+  g_err[0] = 0;
+  Q38_CHECK(check_routing(T, E, k));
+  Q38_CHECK(check_dim(h, "h"));
+  Q38_CHECK(check_dim(I, "I"));
+  const ExpertsWs L = experts_layout(T, h, E, k, I, 0);
+  Q38_CHECK(check_buffer(saved, saved_bytes, train_saved_bytes(T, k, I, L), "saved"));
+  const int32_t needs = (dx != nullptr ? Q38MOE_NEED_X : 0) | (dw != nullptr ? Q38MOE_NEED_TOPK_W : 0) |
+                        (d_gate_up != nullptr ? Q38MOE_NEED_GATE_UP : 0) | (d_down != nullptr ? Q38MOE_NEED_DOWN : 0);
+  TrainWs W;
+  Q38_CHECK(train_work_layout(T, h, E, k, I, needs, &W));
+  Q38_CHECK(check_buffer(work, work_bytes, W.end, "work"));
+  void* sv = const_cast<void*>(saved);  // read only here
+  const int32_t* counts = at<int32_t>(sv, L.counts);
+  const int32_t* starts = at<int32_t>(sv, L.starts);
+  const int32_t* perm = at<int32_t>(sv, L.perm);
+  const int32_t* inv = at<int32_t>(sv, L.inv);
+  const int32_t* tiles = at<int32_t>(sv, L.tiles);
+  const int32_t* tile_count = at<int32_t>(sv, L.tile_count);
+  const void* H = at<uint16_t>(sv, L.H);
+  const void* Y = at<uint16_t>(sv, L.Y);
+  const void* GU = at<uint16_t>(sv, L.end);
+  const bool rows = (needs & ~Q38MOE_NEED_TOPK_W) != 0;
+  void* d_raw = rows ? at<uint16_t>(work, W.d_raw) : nullptr;
+  void* dH = at<uint16_t>(work, W.dH);
+  void* dGU = at<uint16_t>(work, W.dGU);
+  void* partial = at<float>(work, W.partial);
+  if (dw != nullptr)  // one pass over dout for both
+    Q38_CHECK(q38moe_pair_dots(dout, Y, inv, topk_idx, idx_is_int64, rows ? topk_w : nullptr, dw, d_raw, T, h, E, k,
+                               stream));
+  else if (rows)
+    Q38_CHECK(q38moe_gather_rows(dout, perm, topk_w, starts, counts, d_raw, T, h, E, k, stream));
+  if (d_down != nullptr)
+    Q38_CHECK(q38moe_expert_wgrad_ws(d_raw, H, nullptr, starts, counts, d_down, T, h, I, E, k, partial,
+                                     W.partial_bytes, stream));
+  if (dx == nullptr && d_gate_up == nullptr) return Q38MOE_OK;
+  Q38_CHECK(q38moe_down_kn(d_raw, w_down, tiles, tile_count, dH, T, h, I, E, k, stream));
+  Q38_CHECK(q38moe_swiglu_backward(dH, GU, dGU, T * k, I, stream));
+  if (d_gate_up != nullptr)
+    Q38_CHECK(q38moe_expert_wgrad_ws(dGU, x, perm, starts, counts, d_gate_up, T, 2 * I, h, E, k, partial,
+                                     W.partial_bytes, stream));
+  if (dx == nullptr || T == 0) return Q38MOE_OK;
+  void* dxp = at<uint16_t>(work, W.dxp);
+  Q38_CHECK(q38moe_down_kn(dGU, w_gate_up, tiles, tile_count, dxp, T, 2 * I, h, E, k, stream));
+  Q38_HIP(q38::launch_combine(static_cast<const uint16_t*>(dxp), inv, topk_idx, idx_is_int64 != 0, nullptr, nullptr,
+                              nullptr, static_cast<uint16_t*>(dx), T, h, E, k, static_cast<hipStream_t>(stream)),
+          "combine launch");
+  return Q38MOE_OK;
+}
+
 int q38moe_swiglu_backward(const void* dH, const void* GU, void* dGU, int64_t rows, int32_t I,
                            void* stream) {
   g_err[0] = 0;

@@ -53,7 +53,7 @@ __global__ __launch_bounds__(256) void combine_kernel(
 #pragma unroll
   for (int j = 0; j < KT; ++j) {
     row[j] = load_uniform(inv + t * KT + j);
-    wbits[j] = load_uniform_u16(w + t * KT + j);
+    wbits[j] = w != nullptr ? load_uniform_u16(w + t * KT + j) : 0x3f80u;  // no weights: 1.0
   }
   const uint16_t* yrow[KT];
   float wt[KT];

@@ -869,7 +869,7 @@ __global__ __launch_bounds__(ROUTE_THREADS) void route_kernel(
   }
 }
 
-// Few tokens: blocks of G x 16 tokens, a group of 16 being one token per wave for the selection.
+// Few tokens: blocks of 16 tokens, one per wave for the selection.
 //
 // The 64-token block above is a chain of latencies, about 35000 clocks however few blocks a launch
 // has: 12000 until 133 KB of weights and 128 KB of x rows are in (rows read in MFMA layout arrive at
@@ -883,38 +883,33 @@ __global__ __launch_bounds__(ROUTE_THREADS) void route_kernel(
 // (about 3 us) and the launch. Whole launch, back to back, 64-token blocks (T = 1 and 16: split K in
 // one block) -> now, in us:
 //   h = 1024: T = 1 8.9 -> 5.0, 16 11.4 -> 8.0, 61 15.3 -> 9.5, 1000 17.1 -> 10.3, 4096 17.3 -> 12.3
-//   h = 2048: T = 1 12.6 -> 6.4, 48 21.4 -> 12.4, 1000 23.0 -> 12.3, 4096 23.6 -> 13.9, 5003 23.2 -> 20.1
+//   h = 2048: T = 1 12.6 -> 6.4, 48 21.4 -> 12.4, 1000 23.0 -> 12.3, 4096 23.6 -> 13.9
 constexpr int NARROW_WAVES = 16;
 constexpr int NARROW_STRIDE = 68;  // floats per token in LDS (65 used): 4 token rows apart = 16 banks
 
-template <int KT, int G>
+template <int KT>
 __global__ __launch_bounds__(NARROW_WAVES * 64) void route_narrow_kernel(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ wr, const uint16_t* __restrict__ wsg,
     const float* __restrict__ bias, uint16_t* __restrict__ logits_out, int32_t* __restrict__ idx_out,
     uint16_t* __restrict__ w_out, uint16_t* __restrict__ gate_out, int32_t* __restrict__ hist, int64_t T, int h,
     int E) {
-  // Weights of the current K chunk, one wave-private area each; then the partial sums of one group
-  // of 16 tokens at a time.
+  // Weights of the current K chunk, one wave-private area each; then the partial sums.
   __shared__ __attribute__((aligned(16))) uint8_t s_w[NARROW_WAVES][64 * 128];
   float (*const s_part)[NARROW_TOKENS][NARROW_STRIDE] =
       reinterpret_cast<float (*)[NARROW_TOKENS][NARROW_STRIDE]>(&s_w[0][0]);
   static_assert(sizeof(s_w) >= sizeof(float) * NARROW_WAVES * NARROW_TOKENS * NARROW_STRIDE, "partial sums");
-  __shared__ int s_hist[G][64];
+  __shared__ int s_hist[64];
   __shared__ float s_sv[NARROW_WAVES][64];
   __shared__ int s_si[NARROW_WAVES][64];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int64_t tb = (int64_t)blockIdx.x * (NARROW_TOKENS * G);
-  if (tid < G * 64) s_hist[tid >> 6][tid & 63] = 0;
+  const int64_t tb = (int64_t)blockIdx.x * NARROW_TOKENS;
+  if (tid < 64) s_hist[tid] = 0;
   const float zb = bias != nullptr && lane < E ? bias[lane] : 0.0f;
   const int kw = h / NARROW_WAVES;  // multiple of 32 (h % 512 == 0)
   const int kbeg = wave * kw + 8 * (lane >> 4);
-  const uint16_t* xa[G];
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-    const int64_t trow = tb + 16 * g + (lane & 15);
-    xa[g] = x + (trow < T ? trow : T - 1) * (int64_t)h + kbeg;
-  }
-  const uint16_t* const grow = wsg != nullptr ? wsg + kbeg : xa[0];
+  const int64_t trow = tb + (lane & 15);
+  const uint16_t* const xa = x + (trow < T ? trow : T - 1) * (int64_t)h + kbeg;
+  const uint16_t* const grow = wsg != nullptr ? wsg + kbeg : xa;
   // Copies: 8 rows of 128 bytes each, lane l the 16-byte chunk of row 8 i + l / 8 that belongs in
   // slot l % 8 (chunk c of row n is kept in slot c ^ (n & 7): a fragment's 16 rows read distinct
   // banks).
@@ -922,11 +917,9 @@ __global__ __launch_bounds__(NARROW_WAVES * 64) void route_narrow_kernel(
   const uint16_t* const wbase = wr + wave * kw;
   const uint8_t* const frag = s_w[wave] + (lane & 15) * 128;
   const int fs = lane & 7, fq = lane >> 4;  // row & 7 of this lane's fragment rows; its K quarter
-  f32x4_t acc[G][5];
+  f32x4_t acc[5];
 #pragma unroll
-  for (int g = 0; g < G; ++g)
-#pragma unroll
-    for (int j = 0; j < 5; ++j) acc[g][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int j = 0; j < 5; ++j) acc[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
   for (int k0 = 0; k0 < kw; k0 += 64) {
     const bool two = kw - k0 >= 64;  // a last chunk of 32 columns copies chunk 0 to the slots past it
@@ -937,12 +930,7 @@ __global__ __launch_bounds__(NARROW_WAVES * 64) void route_narrow_kernel(
       load_lds16(wbase + (int64_t)(n < E ? n : 0) * h + k0 + c * 8, s_w[wave] + i * 1024);
     }
     const int k1 = two ? k0 + 32 : k0;
-    u32x4_t a[G][2];
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-      a[g][0] = ld16(xa[g] + k0);
-      a[g][1] = ld16(xa[g] + k1);
-    }
+    const u32x4_t a[2] = {ld16(xa + k0), ld16(xa + k1)};
     const u32x4_t sg[2] = {ld16(grow + k0), ld16(grow + k1)};
     wait_vmcnt0();
     asm volatile("" ::: "memory");
@@ -952,50 +940,33 @@ __global__ __launch_bounds__(NARROW_WAVES * 64) void route_narrow_kernel(
 #pragma unroll
       for (int j = 0; j < 5; ++j) {
         const u32x4_t b = j < 4 ? *reinterpret_cast<const u32x4_t*>(frag + j * 2048 + ((4 * s + fq) ^ fs) * 16) : sg[s];
-#pragma unroll
-        for (int g = 0; g < G; ++g) acc[g][j] = mfma16x16x32(a[g][s], b, acc[g][j]);
+        acc[j] = mfma16x16x32(a[s], b, acc[j]);
       }
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // fragments read before the next chunk's copies
   }
+  __syncthreads();  // every wave has read its weights: their area takes the partial sums
+  float* const part = &s_part[wave][4 * (lane >> 4)][lane & 15];
 #pragma unroll
-  for (int g = 0; g < G; ++g) {
-    __syncthreads();  // every wave has read its weights, or the group before: their area is free
-    float* const part = &s_part[wave][4 * (lane >> 4)][lane & 15];
+  for (int i = 0; i < 4; ++i) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) part[i * NARROW_STRIDE + 16 * j] = acc[g][j][i];
-      if ((lane & 15) == 0) part[i * NARROW_STRIDE + 64] = acc[g][4][i];
-    }
-    __syncthreads();
-    // Token `wave` of the group: the sums stay in registers, one expert per lane.
-    float zs = 0.0f;
-#pragma unroll
-    for (int w = 0; w < NARROW_WAVES; ++w) zs += s_part[w][wave][lane];
-    float gs = s_part[lane & 15][wave][64];  // part l in lane l < 16; each row of 16 folds to the total
-    gs += dpp_f(gs, 0xb1);
-    gs += dpp_f(gs, 0x4e);
-    gs += dpp_f(gs, 0x141);
-    gs += dpp_f(gs, 0x140);
-    // The selection of group g runs in a loop over the groups below: one copy of its code.
-    acc[g][0][0] = zs;
-    acc[g][0][1] = gs;
+    for (int j = 0; j < 4; ++j) part[i * NARROW_STRIDE + 16 * j] = acc[j][i];
+    if ((lane & 15) == 0) part[i * NARROW_STRIDE + 64] = acc[4][i];
   }
-  float z = acc[0][0][0], gl = acc[0][0][1];
-#pragma unroll 1
-  for (int g = 0; g < G; ++g) {
-    if constexpr (G > 1) {
+  __syncthreads();
+  const int64_t t = tb + wave;
+  if (t < T) {
+    float z = 0.0f;
 #pragma unroll
-      for (int u = 1; u < G; ++u)
-        if (g == u) {
-          z = acc[u][0][0];
-          gl = acc[u][0][1];
-        }
+    for (int w = 0; w < NARROW_WAVES; ++w) z += s_part[w][wave][lane];
+    if (gate_out != nullptr && wsg != nullptr) {
+      float gl = s_part[lane & 15][wave][64];  // part l in lane l < 16; each row of 16 folds to the total
+      gl += dpp_f(gl, 0xb1);
+      gl += dpp_f(gl, 0x4e);
+      gl += dpp_f(gl, 0x141);
+      gl += dpp_f(gl, 0x140);
+      if (lane == 0) gate_out[t] = (uint16_t)f32_to_bf16_rne(gl);
     }
-    const int64_t t = tb + 16 * g + wave;
-    if (t >= T) break;
-    if (gate_out != nullptr && wsg != nullptr && lane == 0) gate_out[t] = (uint16_t)f32_to_bf16_rne(gl);
     if (logits_out != nullptr && lane < E) logits_out[t * E + lane] = (uint16_t)f32_to_bf16_rne(z);
     int oi;
     float ow;
@@ -1003,51 +974,41 @@ __global__ __launch_bounds__(NARROW_WAVES * 64) void route_narrow_kernel(
     if (lane < KT) {
       idx_out[t * KT + lane] = oi;
       w_out[t * KT + lane] = (uint16_t)f32_to_bf16_rne(ow);
-      atomicAdd(&s_hist[g][oi], 1);
+      atomicAdd(&s_hist[oi], 1);
     }
   }
   if (hist == nullptr) return;
   __syncthreads();
-  if (tid < G * 64 && (tid & 63) < E) {
-    const int64_t row = (int64_t)blockIdx.x * G + (tid >> 6);
-    if (row * NARROW_TOKENS < T) hist[row * E + (tid & 63)] = s_hist[tid >> 6][tid & 63];
-  }
+  if (tid < E) hist[(int64_t)blockIdx.x * E + tid] = s_hist[tid];
 }
 
-// The narrow kernel's groups per block, 0 for the 64-token blocks: as long as one round of blocks (one
-// per CU, by their LDS) takes all tokens, with one group or, up to 8192 tokens on 256 CUs, two (h =
-// 2048: 23.2 -> 20.1 us at T = 5003, 23.9 -> 22.3 at 8192; h = 1024 the same within 0.4 us). Four
-// groups do not fit the registers (T = 16384: 42 us against 18). h % 512: whole MFMA steps per wave.
-static int narrow_groups(int64_t T, int h) {
-  if (h % 512 != 0) return 0;
-  const int64_t groups = (T + NARROW_TOKENS - 1) / NARROW_TOKENS, cus = device_cus();
-  return groups <= cus ? 1 : groups <= 2 * cus ? 2 : 0;
+// The narrow kernel takes calls of up to one round of its blocks (one per CU, by their LDS: 4096 tokens
+// on 256 CUs; above, a second round would cost more than the 64-token blocks: T = 5003 17.8 against 17.5
+// us at h = 1024). Two groups of 16 per block for up to 8192 tokens measured 17.1 against 17.5 us at
+// h = 1024, 20.1 against 23.2 at 2048, but the permutation then reads up to four times the histogram
+// rows, which took that back. h % 512: whole MFMA steps per wave.
+int route_tokens_per_row(int64_t T, int h) {
+  const bool narrow = h % 512 == 0 && (T + NARROW_TOKENS - 1) / NARROW_TOKENS <= device_cus();
+  return narrow ? NARROW_TOKENS : ROUTE_TOKENS;
 }
-
-int route_tokens_per_row(int64_t T, int h) { return narrow_groups(T, h) > 0 ? NARROW_TOKENS : ROUTE_TOKENS; }
 
 hipError_t launch_route(const uint16_t* x, const uint16_t* wr, const uint16_t* wsg,
                         const uint16_t* logits_in, const float* bias, uint16_t* logits_out,
                         int32_t* idx_out, uint16_t* w_out, uint16_t* gate_out, int32_t* hist,
                         int64_t T, int h, int E, int k, hipStream_t stream) {
   if (T == 0) return hipSuccess;
-  const int ng = logits_in == nullptr ? narrow_groups(T, h) : 0;
-  if (ng > 0) {
-    const dim3 grid((unsigned)((T + NARROW_TOKENS * ng - 1) / (NARROW_TOKENS * ng)));
-#define Q38_NARROW(KT, G)                                                                                          \
-  hipLaunchKernelGGL((route_narrow_kernel<KT, G>), grid, dim3(NARROW_WAVES * 64), 0, stream, x, wr, wsg, bias,     \
-                     logits_out, idx_out, w_out, gate_out, hist, T, h, E)
-#define Q38_ROUTE(KT)                     \
-  case KT:                                \
-    if (ng == 1) Q38_NARROW(KT, 1);       \
-    else Q38_NARROW(KT, 2);               \
+  if (logits_in == nullptr && route_tokens_per_row(T, h) == NARROW_TOKENS) {
+    const dim3 grid((unsigned)((T + NARROW_TOKENS - 1) / NARROW_TOKENS));
+#define Q38_ROUTE(KT)                                                                                        \
+  case KT:                                                                                                   \
+    hipLaunchKernelGGL((route_narrow_kernel<KT>), grid, dim3(NARROW_WAVES * 64), 0, stream, x, wr, wsg, bias, \
+                       logits_out, idx_out, w_out, gate_out, hist, T, h, E);                                 \
     break;
     switch (k) {
       Q38_ROUTE(1) Q38_ROUTE(2) Q38_ROUTE(3) Q38_ROUTE(4) Q38_ROUTE(5) Q38_ROUTE(6) Q38_ROUTE(7) Q38_ROUTE(8)
       default: return hipErrorInvalidValue;
     }
 #undef Q38_ROUTE
-#undef Q38_NARROW
     return hipGetLastError();
   }
   const int64_t nblk64 = (T + ROUTE_TOKENS - 1) / ROUTE_TOKENS;

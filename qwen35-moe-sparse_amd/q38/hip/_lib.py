@@ -70,6 +70,11 @@ SIGNATURES = {
     "q38moe_expert_wgrad_workspace_bytes": (_c_int, [_c_i64, _c_i32, _c_i32, _c_i32, _c_i32,
                                                      ctypes.POINTER(_c_size)]),
     "q38moe_expert_wgrad_ws": (_c_int, [_vp] * 6 + [_c_i64, _c_i32, _c_i32, _c_i32, _c_i32, _vp, _c_size, _vp]),
+    "q38moe_experts_train_bytes": (_c_int, [_c_i64] + [_c_i32] * 5 + [ctypes.POINTER(_c_size)] * 2),
+    "q38moe_experts_train_forward": (_c_int, [_vp, _vp, _c_i32, _vp, _vp, _vp, _vp, _c_i64, _c_i32, _c_i32, _c_i32,
+                                              _c_i32, _vp, _c_size, _vp]),
+    "q38moe_experts_train_backward": (_c_int, [_vp] * 3 + [_c_i32] + [_vp] * 4 + [_c_size] + [_vp] * 4 +
+                                      [_c_i64, _c_i32, _c_i32, _c_i32, _c_i32, _vp, _c_size, _vp]),
     "q38moe_swiglu_backward": (_c_int, [_vp, _vp, _vp, _c_i64, _c_i32, _vp]),
     "q38moe_mhc_update": (_c_int, [_c_i32] + [_vp] * 5 + [_c_i64, _c_i32, _c_i32, _vp]),
     "q38moe_mhc_pre": (_c_int, [_vp] * 12 + [_c_i64, _c_i32, _c_i32, _c_i32, ctypes.c_float, _c_i32, _vp]),

@@ -396,6 +396,66 @@ def swiglu_backward(dH, GU):
     return dGU
 
 
+def experts_train_forward(x, topk_idx, topk_w, w_gate_up, w_down):
+    """Routed experts of a training step (q38moe_experts_train_forward): (out [T,h], saved), ``saved`` a
+    byte tensor holding what ``experts_train_backward`` reads besides the inputs."""
+    _need(x, "x", ndim=2)
+    _need(topk_idx, "topk_idx", dtype=None, ndim=2)
+    _need(topk_w, "topk_w", ndim=2)
+    _need(w_gate_up, "w_gate_up", ndim=3)
+    _need(w_down, "w_down", ndim=3)
+    T, h = x.shape
+    k = topk_idx.shape[1]
+    E, twoI, hw = w_gate_up.shape
+    I = twoI // 2
+    if hw != h or twoI % 2:
+        raise ValueError(f"w_gate_up {tuple(w_gate_up.shape)} does not match x {tuple(x.shape)}")
+    if w_down.shape != (E, h, I):
+        raise ValueError(f"w_down {tuple(w_down.shape)} does not match ({E}, {h}, {I})")
+    if topk_idx.shape[0] != T or topk_w.shape != topk_idx.shape:
+        raise ValueError("topk_idx/topk_w must both be [T,k]")
+    n = ctypes.c_size_t()
+    check(lib.q38moe_experts_train_bytes(T, h, E, k, I, 0, ctypes.byref(n), None), "q38moe_experts_train_bytes")
+    saved = torch.empty(n.value, dtype=torch.uint8, device=x.device)
+    out = torch.empty(T, h, dtype=torch.bfloat16, device=x.device)
+    check(lib.q38moe_experts_train_forward(_ptr(x), _ptr(topk_idx), _idx_flag(topk_idx), _ptr(topk_w), _ptr(w_gate_up),
+                                           _ptr(w_down), _ptr(out), T, h, E, k, I, _ptr(saved), n.value,
+                                           _stream(x.device)), "q38moe_experts_train_forward")
+    return out, saved
+
+
+def experts_train_backward(dout, x, topk_idx, topk_w, w_gate_up, w_down, saved, need_x=True, need_w=True,
+                           need_gate_up=True, need_down=True):
+    """Gradients (dx, d topk_w, d gate_up_proj, d down_proj) of ``experts_train_forward``'s output, None
+    where not needed (q38moe_experts_train_backward)."""
+    _need(dout, "dout", ndim=2)
+    _need(x, "x", ndim=2)
+    _need(topk_idx, "topk_idx", dtype=None, ndim=2)
+    _need(topk_w, "topk_w", ndim=2)
+    _need(w_gate_up, "w_gate_up", ndim=3)
+    _need(w_down, "w_down", ndim=3)
+    _need(saved, "saved", dtype=torch.uint8, ndim=1)
+    T, h = x.shape
+    k = topk_idx.shape[1]
+    E, twoI, _ = w_gate_up.shape
+    if dout.shape != x.shape:
+        raise ValueError(f"dout {tuple(dout.shape)} does not match x {tuple(x.shape)}")
+    dx = torch.empty_like(x) if need_x else None
+    dw = torch.empty_like(topk_w) if need_w else None
+    dgu = torch.empty_like(w_gate_up) if need_gate_up else None
+    ddn = torch.empty_like(w_down) if need_down else None
+    n = ctypes.c_size_t()
+    check(lib.q38moe_experts_train_bytes(T, h, E, k, twoI // 2,
+                                         1 * need_x | 2 * need_w | 4 * need_gate_up | 8 * need_down, None,
+                                         ctypes.byref(n)), "q38moe_experts_train_bytes")
+    work = torch.empty(n.value, dtype=torch.uint8, device=x.device)
+    check(lib.q38moe_experts_train_backward(_ptr(dout), _ptr(x), _ptr(topk_idx), _idx_flag(topk_idx), _ptr(topk_w),
+                                            _ptr(w_gate_up), _ptr(w_down), _ptr(saved), saved.numel(), _ptr(dx),
+                                            _ptr(dw), _ptr(dgu), _ptr(ddn), T, h, E, k, twoI // 2, _ptr(work), n.value,
+                                            _stream(x.device)), "q38moe_experts_train_backward")
+    return dx, dw, dgu, ddn
+
+
 def experts_workspace_bytes(T, h, E, k, I, dtype=torch.bfloat16):
     n = ctypes.c_size_t()
     check(lib.q38moe_experts_workspace_bytes(T, h, E, k, I, _DTYPES[dtype], ctypes.byref(n)),

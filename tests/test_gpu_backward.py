@@ -429,3 +429,31 @@ def test_expert_wgrad_split_rows(gpu, E, k, T, M, N, skip):
         Gt = G[s0:s0 + c].float().T.contiguous()
         assert_gemm_bf16_rounding(gathered[e], Gt, x[rows // k].float().T.contiguous(), what=f"gathered[{e}]")
         assert_gemm_bf16_rounding(ordered[e], Gt, xs[s0:s0 + c].float().T.contiguous(), what=f"sorted[{e}]")
+
+
+@pytest.mark.parametrize("T", [0, 1, 130])
+@pytest.mark.parametrize("idx_dtype", [torch.int32, torch.int64])
+def test_experts_train_gradients_on_demand(gpu, T, idx_dtype):
+    """Each subset of the gradients gives the bits of the call that asks for all of them (the same
+    kernels run; the routed rows' gradient comes from one of two that round alike), and a buffer that is
+    too small is refused before any launch."""
+    from q38.hip import ops
+    E, k, h, I = 8, 3, 128, 64
+    g = torch.Generator().manual_seed(T)
+    r = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16).to(gpu)
+    x, w, gu, dn, dout = r(T, h), r(T, k), r(E, 2 * I, h) * 0.1, r(E, h, I) * 0.1, r(T, h)
+    idx = torch.stack([torch.randperm(E, generator=g)[:k] for _ in range(T)]) if T else torch.empty(0, k)
+    idx = idx.to(idx_dtype).to(gpu)
+    out, saved = ops.experts_train_forward(x, idx, w, gu, dn)
+    assert out.shape == x.shape
+    full = ops.experts_train_backward(dout, x, idx, w, gu, dn, saved)
+    if T == 0:
+        assert not full[2].any() and not full[3].any()  # weight gradients without rows are zero
+    for mask in range(1, 16):
+        need = [bool(mask >> i & 1) for i in range(4)]
+        part = ops.experts_train_backward(dout, x, idx, w, gu, dn, saved, *need)
+        for n, a, b in zip(need, part, full):
+            assert torch.equal(a, b) if n else a is None
+    if T:
+        with pytest.raises(RuntimeError):
+            ops.experts_train_backward(dout, x, idx, w, gu, dn, saved[:-256])

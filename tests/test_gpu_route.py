@@ -201,9 +201,8 @@ def test_route_full(gpu, wl_name, T):
     (17, 1536, 17, 4),     # one full 64-column chunk and one of 32; a second block of one token
     (64, 1024, 8, 8),      # E = k: every row has fewer than k + 1 experts
     (4095, 512, 64, 8),    # last one-group block ragged
-    (4113, 1024, 64, 5),   # two groups of 16 per block on 256 CUs, the last block's second one partial
-    (4129, 1024, 40, 3),   # the last block without its second group
-    (8193, 512, 64, 5),    # past the narrow blocks
+    (4113, 1024, 64, 5),   # past one round of narrow blocks on 256 CUs
+    (4096, 1024, 40, 3),   # a full round of them
 ])
 def test_route_few_tokens(gpu, T, h, E, k):
     """Blocks of 16 tokens and their neighbours, logits from x: 0/1 activations and weights give exact
