@@ -84,9 +84,19 @@ __global__ __launch_bounds__(256) void permute_kernel(
         if (bb + 4 * u < b) bef += c[u];
       }
     }
-    // The rest, 64 rows a step: loads past the last row repeat it and count nothing (one round trip;
-    // one row at a time, the 15 rows of a part cost about 3 us).
-    for (; bb < nblk; bb += 64) {
+    for (; bb + 60 < nblk; bb += 64) {
+      int c[16];
+#pragma unroll
+      for (int u = 0; u < 16; ++u) c[u] = hist[(int64_t)(bb + 4 * u) * E + e];
+#pragma unroll
+      for (int u = 0; u < 16; ++u) {
+        tot += c[u];
+        if (bb + 4 * u < b) bef += c[u];
+      }
+    }
+    // The last rows: loads past the end repeat the last one and count nothing (one round trip; one row
+    // at a time, the 15 rows of a part cost about 3 us).
+    if (bb < nblk) {
       int c[16];
 #pragma unroll
       for (int u = 0; u < 16; ++u) c[u] = hist[(int64_t)min(bb + 4 * u, nblk - 1) * E + e];
