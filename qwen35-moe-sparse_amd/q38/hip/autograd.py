@@ -115,8 +115,30 @@ def router_backward(x, w_router, logits, idx, bias, d_logits, d_w, need_x=True, 
         return None, None
     dz = dz.to(logits.dtype)
     dx = dz @ w_router if need_x else None
-    dwr = dz.t().contiguous() @ x if need_w else None
-    return dx, dwr
+    return dx, _router_weight_grad(dz, x) if need_w else None
+
+
+def _eager(*tensors):
+    """True when nothing records, batches or traces the call and the tensors are plain ones."""
+    return (not torch.is_grad_enabled() and torch._C._functorch.peek_interpreter_stack() is None
+            and not torch.compiler.is_compiling() and all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in tensors))
+
+
+def _router_weight_grad(dz, x):
+    """dz^T . x [E, h]. From 6144 bf16 tokens on the GPU the expert weight-gradient kernel takes it as one
+    expert that holds every row: its blocks split the rows, where the library's product of 64 output rows
+    leaves most of the chip idle (hidden 512 to 1024, library and this in us: T = 4096 25 and 28, 8192 44
+    and 28, 16384 85 to 111 and 29; the same error against float64). Below, the two small tensors cost the
+    host more than that gains. With a graph of the gradient itself (create_graph), under vmap or tracing,
+    and for other types and widths, torch's product."""
+    T, h = x.shape
+    E = dz.shape[1]
+    if (x.is_cuda and x.dtype == dz.dtype == torch.bfloat16 and T >= 6144 and E % 64 == 0 and h % 64 == 0
+            and 2 * T * max(E, h) < 2**31 and _eager(dz, x)):
+        starts = torch.zeros(1, dtype=torch.int32, device=x.device)
+        counts = torch.full((1,), T, dtype=torch.int32, device=x.device)
+        return ops.expert_wgrad(dz.contiguous(), x.contiguous(), starts, counts, 1)[0]
+    return dz.t().contiguous() @ x
 
 
 def router(x, w_router, k, logit_bias=None):

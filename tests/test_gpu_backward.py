@@ -457,3 +457,19 @@ def test_experts_train_gradients_on_demand(gpu, T, idx_dtype):
     if T:
         with pytest.raises(RuntimeError):
             ops.experts_train_backward(dout, x, idx, w, gu, dn, saved[:-256])
+
+
+@pytest.mark.parametrize("T,E,h", [(6143, 64, 1024), (6144, 64, 1024), (6159, 64, 320), (9001, 128, 64), (6144, 60, 256)])
+def test_router_weight_grad(gpu, T, E, h):
+    """The router's weight gradient on both sides of its dispatch (6144 tokens, multiples of 64) against
+    float64: one bf16 rounding plus an fp32 sum of T exact products, at most T 2^-24 of their magnitudes."""
+    from q38.hip import autograd
+    g = torch.Generator().manual_seed(T + E)
+    dz = (torch.randn(T, E, generator=g) * 0.01).to(torch.bfloat16).to(gpu)
+    x = torch.randn(T, h, generator=g).to(torch.bfloat16).to(gpu)
+    with torch.no_grad():
+        got = autograd._router_weight_grad(dz, x)
+    exact = dz.double().t() @ x.double()
+    bound = exact.abs() * 2.0**-8 + T * 2.0**-24 * (dz.double().abs().t() @ x.double().abs())
+    assert got.shape == (E, h) and got.dtype == torch.bfloat16
+    assert bool(((got.double() - exact).abs() <= bound).all())
