@@ -40,9 +40,11 @@ __global__ __launch_bounds__(256) void combine_kernel(
   if (t >= T) return;
   // Routing entries of the token's pairs p = t*k + j; a pair whose index lies outside [0, E) is
   // dropped (its row is never read).
+  // Without weights (1.0 each) the loads go to inv and are not used: no branch between the loads.
   int64_t ev[KT];
   int32_t row[KT];
   uint32_t wbits[KT];
+  const uint16_t* const wsrc = w != nullptr ? w : reinterpret_cast<const uint16_t*>(inv);
   if (idx != nullptr) {
 #pragma unroll
     for (int j = 0; j < KT; ++j) ev[j] = (int64_t)load_uniform(idx + t * KT + j);
@@ -53,7 +55,8 @@ __global__ __launch_bounds__(256) void combine_kernel(
 #pragma unroll
   for (int j = 0; j < KT; ++j) {
     row[j] = load_uniform(inv + t * KT + j);
-    wbits[j] = w != nullptr ? load_uniform_u16(w + t * KT + j) : 0x3f80u;  // no weights: 1.0
+    const uint32_t bits = load_uniform_u16(wsrc + t * KT + j);
+    wbits[j] = w != nullptr ? bits : 0x3f80u;
   }
   const uint16_t* yrow[KT];
   float wt[KT];

@@ -7,6 +7,8 @@
 // perm[starts[e] + r] = the r-th pair (ascending p) routed to e. Every block of 64 tokens derives
 // its base offsets from the per-block histograms, so the scatter needs no atomics and the order is
 // deterministic.
+#include <type_traits>
+
 #include "q38moe_common.h"
 #include "q38moe_kernels.h"
 
@@ -94,18 +96,21 @@ __global__ __launch_bounds__(256) void permute_kernel(
         if (bb + 4 * u < b) bef += c[u];
       }
     }
-    // The last rows: loads past the end repeat the last one and count nothing (one round trip; one row
-    // at a time, the 15 rows of a part cost about 3 us).
-    if (bb < nblk) {
-      int c[16];
+    // The last rows: loads past the end repeat the last one and count nothing, all in one round trip
+    // (one row at a time, the 15 rows of a part cost about 3 us; a few rows take the short form).
+    auto rest = [&](auto n) {
+      constexpr int R = decltype(n)::value;
+      int c[R];
 #pragma unroll
-      for (int u = 0; u < 16; ++u) c[u] = hist[(int64_t)min(bb + 4 * u, nblk - 1) * E + e];
+      for (int u = 0; u < R; ++u) c[u] = hist[(int64_t)min(bb + 4 * u, nblk - 1) * E + e];
 #pragma unroll
-      for (int u = 0; u < 16; ++u) {
+      for (int u = 0; u < R; ++u) {
         if (bb + 4 * u < nblk) tot += c[u];
         if (bb + 4 * u < b && bb + 4 * u < nblk) bef += c[u];
       }
-    }
+    };
+    if (bb + 4 < nblk) rest(std::integral_constant<int, 16>{});
+    else if (bb < nblk) rest(std::integral_constant<int, 1>{});
   }
   s_tot[part][e] = tot;
   s_bef[part][e] = bef;
