@@ -1310,7 +1310,8 @@ int q38moe_mhc_update(int32_t mode, float* X, const void* y, const float* post, 
   Q38_CHECK(check_dtype(dtype));
   Q38_CHECK(check_dim(h, "h"));
   if (mode < Q38MOE_MHC_INIT || mode > Q38MOE_MHC_POST) return fail(Q38MOE_EINVAL, "unknown mode %d", mode);
-  if (T < 0 || T >= (int64_t)1 << 31) return fail(Q38MOE_EINVAL, "T must be in [0, 2^31)");
+  if (T < 0 || T >= (int64_t)1 << 24)  // one block of 256 threads per token
+    return fail(Q38MOE_EINVAL, "T must be in [0, 2^24)");
   if (T == 0) return Q38MOE_OK;
   Q38_CHECK(check_ptr(X, "X"));
   Q38_CHECK(check_ptr(y, "y"));

@@ -564,13 +564,18 @@ def _mhc_post(X, y, state):
 
 def _native_trunk(M, cfg, ids):
     """True when the trunk's own kernels (q38.hip.ops.mhc_*, gdn_*, qsa_*) take this forward: tokens and parameters
-    plain tensors on one GPU, parameters all bf16 or all fp32 and contiguous, no gradient, tracing or
-    function transform to record, and the shapes they are built for. Otherwise the torch code runs."""
+    plain tensors on the current GPU, parameters all bf16 or all fp32 and contiguous, no gradient, autocast,
+    tracing or function transform in force, and the shapes they are built for. Otherwise the torch code runs.
+    Gradients by mode and not by the parameters: the MoE callable may hold parameters of its own."""
     from torch.autograd import forward_ad
 
     if not ids.is_cuda or type(ids) is not torch.Tensor or cfg.n_branch != 4:
         return False
+    if ids.device.index != torch.cuda.current_device() or ids.numel() >= 2 ** 24:  # one block of 256 per token
+        return False
     if cfg.hidden % 64 or cfg.hidden > 2048 or cfg.mhc_rank % 4 or cfg.mhc_rank > 128:
+        return False
+    if torch.is_grad_enabled() or torch.is_autocast_enabled("cuda"):
         return False
     if torch.jit.is_tracing() or torch.compiler.is_compiling() or forward_ad._current_level >= 0:
         return False
@@ -579,8 +584,7 @@ def _native_trunk(M, cfg, ids):
     dt = M.embed_tokens.weight.dtype
     if dt not in (torch.bfloat16, torch.float32):
         return False
-    grad = torch.is_grad_enabled()
-    return all(p.dtype == dt and p.device == ids.device and p.is_contiguous() and not (grad and p.requires_grad)
+    return all(p.dtype == dt and p.device == ids.device and p.is_contiguous()
                and type(p) in (torch.Tensor, nn.Parameter) for p in M.parameters())
 
 

@@ -191,8 +191,18 @@ def test_trunk_choice(gpu):
     ids = torch.arange(70, device=gpu)[None] % 128
     model = P.build(cfg, device=gpu, dtype=torch.float32, moe_forward=lambda block, x: 0.1 * x)
     M = model.model
-    assert P._native_trunk(M, cfg, ids) and not P._native_trunk(M, cfg, ids.cpu())
+    with torch.no_grad():
+        assert P._native_trunk(M, cfg, ids) and not P._native_trunk(M, cfg, ids.cpu())
     native = model(ids)
+    # A trainable MoE callable over frozen parameters gets its gradient.
+    scale = torch.tensor(0.1, device=gpu, requires_grad=True)
+    P.trunk_forward(M, cfg, ids, lambda block, x, r: scale * x).square().mean().backward()
+    assert float(scale.grad.abs()) > 0
+    # Autocast hands the mixers bf16 activations beside fp32 parameters: the torch code takes them (bf16
+    # products, 2^-8 each, through a dozen of them in a row).
+    with torch.autocast("cuda", torch.bfloat16):
+        cast = model(ids)
+    assert _rel(cast.float(), native.double()) < 12 * 2**-8
     M.requires_grad_(True)
     assert not P._native_trunk(M, cfg, ids)
     hs = P.trunk_forward(M, cfg, ids, lambda block, x, r: 0.1 * x)
