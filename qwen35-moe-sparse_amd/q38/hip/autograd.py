@@ -28,6 +28,7 @@ the output comes back in hidden_states' dtype, so their gradients arrive in thei
 are int32/int64 as in the forward.
 """
 import torch
+from torch.autograd import forward_ad
 
 from . import ops
 
@@ -119,8 +120,10 @@ def router_backward(x, w_router, logits, idx, bias, d_logits, d_w, need_x=True, 
 
 
 def _eager(*tensors):
-    """True when nothing records, batches or traces the call and the tensors are plain ones."""
-    return (not torch.is_grad_enabled() and torch._C._functorch.peek_interpreter_stack() is None
+    """True when nothing records, batches, traces or carries tangents through the call and the tensors are
+    plain ones."""
+    return (not torch.is_grad_enabled() and forward_ad._current_level < 0
+            and torch._C._functorch.peek_interpreter_stack() is None and not torch.jit.is_tracing()
             and not torch.compiler.is_compiling() and all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in tensors))
 
 

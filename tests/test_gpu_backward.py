@@ -10,6 +10,7 @@ The forward output keeps the forward tolerance (tests/_util.py).
 """
 import pytest
 import torch
+from torch.autograd import forward_ad
 
 from _util import assert_bf16_close, assert_gemm_bf16_rounding
 from oracle import moe_oracle as orc
@@ -473,3 +474,8 @@ def test_router_weight_grad(gpu, T, E, h):
     bound = exact.abs() * 2.0**-8 + T * 2.0**-24 * (dz.double().abs().t() @ x.double().abs())
     assert got.shape == (E, h) and got.dtype == torch.bfloat16
     assert bool(((got.double() - exact).abs() <= bound).all())
+    # Forward-mode tangents pass through the product: with dz as its own tangent, the product itself.
+    with torch.no_grad(), forward_ad.dual_level():
+        out = autograd._router_weight_grad(forward_ad.make_dual(dz, dz), x)
+        tangent = forward_ad.unpack_dual(out).tangent
+    assert tangent is not None and bool(((tangent.double() - exact).abs() <= bound).all())
