@@ -1369,7 +1369,7 @@ int q38moe_gdn_conv(const void* qkv, const void* conv_w, void* out, int64_t B, i
   Q38_CHECK(check_dim(C, "C"));
   if (B < 0 || S < 0 || B * (int64_t)S >= (int64_t)1 << 31) return fail(Q38MOE_EINVAL, "bad B or S");
   if (B == 0 || S == 0) return Q38MOE_OK;
-  if ((B * ((S + 7) / 8) * (int64_t)(C / 4) + 255) / 256 >= (int64_t)1 << 31)
+  if (B * ((S + 7) / 8) * (int64_t)(C / 4) + 255 >= (int64_t)1 << 32)  // 32-bit thread ids, 32 elements each
     return fail(Q38MOE_EINVAL, "B * S * C is too large");
   Q38_CHECK(check_ptr(qkv, "qkv"));
   Q38_CHECK(check_ptr(conv_w, "conv_w"));

@@ -231,25 +231,29 @@ __global__ __launch_bounds__(256) void mhc_pre_kernel(const float* __restrict__ 
 
 // Causal depthwise convolution of 4 taps in fp32, rounded to dt, then SiLU rounded to dt
 // (modeling:184-205): qkv, out [B, S, C]. A thread owns 4 channels and GDN_TS consecutive steps (a
-// sliding window of rows in registers); products and sums are rounded one by one. HBM-bound: 105 us for
-// 273 MB at 16384 x 4160 (as torch operations on transposed fp32 copies some 1.2 ms).
+// sliding window of rows in registers); products and sums are rounded one by one. 273 MB at 16384 x 4160 in
+// bf16 take 101 us in a prefill and 88-92 us alone (3 TB/s, below the copy rate; as torch operations on
+// transposed fp32 copies some 1.2 ms): arithmetic next to the loads, so that 32-bit thread ids and one
+// conversion per two roundings gained (107 -> 101 us, 1024 x 4160 alone 10.6 -> 10.0, 64 x 192 5.7 -> 5.2).
+// 8 channels per thread by 16-byte loads: 81 us at the first of these, but 12.5 and 7.2 us at the others
+// (too few threads) and fp32 103 -> 122 us.
 constexpr int GDN_TS = 8;
 
 template <bool BF16>
 __global__ __launch_bounds__(256) void gdn_conv_kernel(const void* __restrict__ qkv, const void* __restrict__ w,
-                                                       void* __restrict__ out, int64_t runs, int S, int C) {
-  const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int cq = C / 4;
-  const int64_t run = id / cq;  // (sequence, run of GDN_TS steps)
+                                                       void* __restrict__ out, uint32_t runs, int S, int C) {
+  const uint32_t id = blockIdx.x * 256u + threadIdx.x;
+  const uint32_t cq = (uint32_t)C / 4;
+  const uint32_t run = id / cq;  // (sequence, run of GDN_TS steps)
   if (run >= runs) return;
   const int c = 4 * (int)(id - run * cq);
-  const int per_seq = (S + GDN_TS - 1) / GDN_TS;
-  const int64_t b = run / per_seq;
+  const uint32_t per_seq = (uint32_t)(S + GDN_TS - 1) / GDN_TS;
+  const uint32_t b = run / per_seq;
   const int s0 = (int)(run - b * per_seq) * GDN_TS;
   f32x4_t taps[4];  // taps[i]: the four taps of channel c + i
 #pragma unroll
   for (int i = 0; i < 4; ++i) taps[i] = ld4_dt<BF16>(w, 4 * (int64_t)(c + i));
-  const int64_t base = b * S * C + c;
+  const int64_t base = (int64_t)b * S * C + c;
   f32x4_t x[3 + GDN_TS];
 #pragma unroll
   for (int j = 0; j < 3 + GDN_TS; ++j) {
@@ -262,10 +266,16 @@ __global__ __launch_bounds__(256) void gdn_conv_kernel(const void* __restrict__ 
     f32x4_t y;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      float a = __fmul_rn(x[j][i], taps[i][0]);
+      y[i] = __fmul_rn(x[j][i], taps[i][0]);
 #pragma unroll
-      for (int k = 1; k < 4; ++k) a = __fadd_rn(a, __fmul_rn(x[j + k][i], taps[i][k]));
-      y[i] = silu_f32(round_dt<BF16>(a));
+      for (int k = 1; k < 4; ++k) y[i] = __fadd_rn(y[i], __fmul_rn(x[j + k][i], taps[i][k]));
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i += 2) {
+      float lo = y[i], hi = y[i + 1];
+      if (BF16) unpack_bf16x2(pack_bf16x2(lo, hi), lo, hi);  // both rounded by one instruction
+      y[i] = silu_f32(lo);
+      y[i + 1] = silu_f32(hi);
     }
     st4_dt<BF16>(out, base + (int64_t)(s0 + j) * C, y);
   }
@@ -918,9 +928,10 @@ hipError_t launch_gdn_conv(const void* qkv, const void* w, void* out, int64_t B,
                            hipStream_t stream) {
   const int64_t runs = B * ((S + GDN_TS - 1) / GDN_TS);
   if (runs == 0) return hipSuccess;
+  if (runs * (C / 4) + 255 >= (int64_t)1 << 32) return hipErrorInvalidValue;  // 32-bit thread ids
   const dim3 grid((unsigned)((runs * (C / 4) + 255) / 256));
-  if (bf16) hipLaunchKernelGGL(gdn_conv_kernel<true>, grid, dim3(256), 0, stream, qkv, w, out, runs, S, C);
-  else hipLaunchKernelGGL(gdn_conv_kernel<false>, grid, dim3(256), 0, stream, qkv, w, out, runs, S, C);
+  if (bf16) hipLaunchKernelGGL(gdn_conv_kernel<true>, grid, dim3(256), 0, stream, qkv, w, out, (uint32_t)runs, S, C);
+  else hipLaunchKernelGGL(gdn_conv_kernel<false>, grid, dim3(256), 0, stream, qkv, w, out, (uint32_t)runs, S, C);
   return hipGetLastError();
 }
 
