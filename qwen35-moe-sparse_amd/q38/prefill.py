@@ -750,8 +750,8 @@ def trunk_forward(M, cfg, ids, moe, router=None):
     if native:
         from .hip import ops
 
-        X = torch.empty(B, S, cfg.n_branch, cfg.hidden, device=ids.device)
-        ssq = torch.empty(B * S, device=ids.device)
+        X = torch.empty(B, S, cfg.n_branch, cfg.hidden, dtype=torch.float32, device=ids.device)
+        ssq = torch.empty(B * S, dtype=torch.float32, device=ids.device)
         Xt = X.view(B * S, cfg.n_branch, cfg.hidden)
         ops.mhc_update(ops.MHC_INIT, Xt, e.view(B * S, cfg.hidden), ssq)
     else:

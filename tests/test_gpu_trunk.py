@@ -215,3 +215,24 @@ def test_trunk_choice(gpu):
         assert not P._native_trunk(M, cfg, ids)
         M.norm.to(torch.float32)
     assert _rel(native, (hs @ M.embed_tokens.weight.t()).detach().double()) < 1e-5
+
+
+def _small_model(gpu, moe_forward=lambda block, x: 0.1 * x):
+    """A period of the layer pattern in fp32, with 70 tokens."""
+    cfg = P.PrefillConfig(vocab=128, hidden=128, layers=4, heads=4, kv_heads=2, lin_k_heads=1, lin_v_heads=2,
+                          moe_ffn=64, shared_ffn=64, ngram_rows=64, experts=8, topk=2)
+    model = P.build(cfg, device=gpu, dtype=torch.float32, moe_forward=moe_forward)
+    return cfg, model, torch.arange(70, device=gpu)[None] % 128
+
+
+@pytest.mark.parametrize("default", [torch.bfloat16, torch.float64])
+def test_trunk_default_dtype(gpu, default):
+    """The stream is fp32 whatever torch's default dtype is."""
+    _, model, ids = _small_model(gpu)
+    expected = model(ids)
+    torch.set_default_dtype(default)
+    try:
+        got = model(ids)
+    finally:
+        torch.set_default_dtype(torch.float32)
+    assert torch.equal(got, expected)
