@@ -564,8 +564,9 @@ def _mhc_post(X, y, state):
 
 def _native_trunk(M, cfg, ids):
     """True when the trunk's own kernels (q38.hip.ops.mhc_*, gdn_*, qsa_*) take this forward: tokens and parameters
-    plain tensors on the current GPU, parameters all bf16 or all fp32 and contiguous, no gradient, autocast,
-    tracing or function transform in force, and the shapes they are built for. Otherwise the torch code runs.
+    plain tensors on the current GPU, parameters all bf16 or all fp32, contiguous and on 16-byte boundaries (views
+    into a flat buffer need not be), no gradient, autocast, tracing or function transform in force, and the shapes
+    they are built for. Otherwise the torch code runs.
     Gradients by mode and not by the parameters: the MoE callable may hold parameters of its own."""
     from torch.autograd import forward_ad
 
@@ -584,7 +585,7 @@ def _native_trunk(M, cfg, ids):
     dt = M.embed_tokens.weight.dtype
     if dt not in (torch.bfloat16, torch.float32):
         return False
-    return all(p.dtype == dt and p.device == ids.device and p.is_contiguous()
+    return all(p.dtype == dt and p.device == ids.device and p.is_contiguous() and p.data_ptr() % 16 == 0
                and type(p) in (torch.Tensor, nn.Parameter) for p in M.parameters())
 
 

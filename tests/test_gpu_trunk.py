@@ -236,3 +236,24 @@ def test_trunk_default_dtype(gpu, default):
     finally:
         torch.set_default_dtype(torch.float32)
     assert torch.equal(got, expected)
+
+
+def _off_boundary(t):
+    """A contiguous copy of t that does not start on a 16-byte boundary: a view into a flat buffer."""
+    v = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)[1:].view(t.shape)
+    assert v.is_contiguous() and v.data_ptr() % 16
+    return v.copy_(t)
+
+
+@pytest.mark.parametrize("name", ["layers.0.input_layernorm.weight", "layers.0.linear_attn.conv1d.weight",
+                                  "layers.0.linear_attn.norm.weight", "layers.3.self_attn.q_norm.weight",
+                                  "layers.3.self_attn.k_norm.weight"])
+def test_trunk_unaligned_parameter(gpu, name):
+    """A parameter that is a view into a flat buffer takes the torch code, which needs no alignment."""
+    cfg, model, ids = _small_model(gpu)
+    expected = model(ids)
+    p = model.model.get_parameter(name)
+    p.data = _off_boundary(p.data)
+    with torch.no_grad():
+        assert not P._native_trunk(model.model, cfg, ids)
+    assert _rel(model(ids), expected.double()) < 1e-5
