@@ -257,3 +257,11 @@ def test_trunk_unaligned_parameter(gpu, name):
     with torch.no_grad():
         assert not P._native_trunk(model.model, cfg, ids)
     assert _rel(model(ids), expected.double()) < 1e-5
+
+
+def test_trunk_unaligned_moe_output(gpu):
+    """The MoE callable's output may be any view."""
+    _, model, ids = _small_model(gpu)
+    expected = model(ids)
+    model.moe_forward = lambda block, x: _off_boundary(0.1 * x)
+    assert torch.equal(model(ids), expected)
