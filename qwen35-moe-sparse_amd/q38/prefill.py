@@ -613,7 +613,7 @@ def _mhc_out(X, y, state, ssq):
     B, S, n, h = X.shape
     if y.dtype not in (torch.bfloat16, torch.float32):
         y = y.float()
-    y = y.reshape(B * S, h).contiguous()
+    y = y.expand(B, S, h).reshape(B * S, h).contiguous()
     if y.data_ptr() % 16:  # the MoE callable may return a view of a buffer of its own
         y = y.clone()
     ops.mhc_update(ops.MHC_POST, X.view(B * S, n, h), y, ssq, *state)

@@ -265,3 +265,13 @@ def test_trunk_unaligned_moe_output(gpu):
     expected = model(ids)
     model.moe_forward = lambda block, x: _off_boundary(0.1 * x)
     assert torch.equal(model(ids), expected)
+
+
+def test_trunk_broadcast_moe_output(gpu):
+    """The MoE callable's output may be broadcast over tokens or features, as the torch code's products take it."""
+    _, model, ids = _small_model(gpu)
+    for dims in ((-1,), (1,), (0, 1, 2)):
+        model.moe_forward = lambda block, x: x.mean(dims, keepdim=True)
+        got = model(ids)
+        model.moe_forward = lambda block, x: x.mean(dims, keepdim=True).expand_as(x).contiguous()
+        assert torch.equal(got, model(ids))
