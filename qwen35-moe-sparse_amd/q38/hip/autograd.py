@@ -133,14 +133,17 @@ def _router_weight_grad(dz, x):
     leaves most of the chip idle (hidden 512 to 1024, library and this in us: T = 4096 25 and 28, 8192 44
     and 28, 16384 85 to 111 and 29; the same error against float64). Below, the two small tensors cost the
     host more than that gains. With a graph of the gradient itself (create_graph), under vmap or tracing,
-    and for other types and widths, torch's product."""
+    for other types and widths, and for rows off 16-byte boundaries or on another than the current GPU,
+    torch's product."""
     T, h = x.shape
     E = dz.shape[1]
     if (x.is_cuda and x.dtype == dz.dtype == torch.bfloat16 and T >= 6144 and E % 64 == 0 and h % 64 == 0
-            and 2 * T * max(E, h) < 2**31 and _eager(dz, x)):
-        starts = torch.zeros(1, dtype=torch.int32, device=x.device)
-        counts = torch.full((1,), T, dtype=torch.int32, device=x.device)
-        return ops.expert_wgrad(dz.contiguous(), x.contiguous(), starts, counts, 1)[0]
+            and 2 * T * max(E, h) < 2**31 and x.device.index == torch.cuda.current_device() and _eager(dz, x)):
+        dz, x = dz.contiguous(), x.contiguous()
+        if dz.data_ptr() % 16 == 0 and x.data_ptr() % 16 == 0:
+            starts = torch.zeros(1, dtype=torch.int32, device=x.device)
+            counts = torch.full((1,), T, dtype=torch.int32, device=x.device)
+            return ops.expert_wgrad(dz, x, starts, counts, 1)[0]
     return dz.t().contiguous() @ x
 
 
