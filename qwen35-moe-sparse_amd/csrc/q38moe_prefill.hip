@@ -121,7 +121,8 @@ __global__ __launch_bounds__(256) void mhc_update_kernel(float* X, const void* _
 // Sublayer input and mixing coefficients (modeling:994-1031 and the zero-centred norm, :839-853) of TPB
 // tokens per block: z = tanh((z0 r) B^T) with r the RMS factor of the token's 4 h values; pre =
 // sigmoid(b_pre + a0 z), post = 2 sigmoid(b_post + a1 z); the 4 x 4 residual mix is Sinkhorn-normalised,
-// sixteen lanes per token, one element each (row sums over lanes ^ 1, ^ 2, column sums over ^ 4, ^ 8).
+// sixteen lanes per token, one element each (row sums over lanes ^ 1, ^ 2, column sums over ^ 4, ^ 8). Its
+// maximum and clamped sums keep a NaN, as torch's amax and clamp do (v_maximum3_f32; fmaxf would drop it).
 // Then, one wave per token: xin = sum_b pre_b X_b, x = dt(xin / rms(xin) (1 + w)). 16 tokens per block
 // keep every lane of the coefficient phase busy; 4 spread short prompts over the chip.
 template <int TPB, int NCH, bool BF16>
@@ -171,15 +172,15 @@ __global__ __launch_bounds__(256) void mhc_pre_kernel(const float* __restrict__ 
     float l = ld_dt<BF16>(b_res, j) + ld_dt<BF16>(alphas, 2) * zr;
     float m = l;
 #pragma unroll
-    for (int o = 1; o < 16; o <<= 1) m = fmaxf(m, __shfl_xor(m, o));
+    for (int o = 1; o < 16; o <<= 1) m = __builtin_elementwise_maximum(m, __shfl_xor(m, o));
     float v = expf(l - m);
     for (int it = 0; it < iters; ++it) {
       float s = v + __shfl_xor(v, 1);
       s += __shfl_xor(s, 2);
-      v = v / fmaxf(s, 1e-9f);
+      v = v / __builtin_elementwise_maximum(s, 1e-9f);
       s = v + __shfl_xor(v, 4);
       s += __shfl_xor(s, 8);
-      v = v / fmaxf(s, 1e-9f);
+      v = v / __builtin_elementwise_maximum(s, 1e-9f);
     }
     if (t < T) P[t * 16 + j] = v;
   }

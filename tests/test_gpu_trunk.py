@@ -275,3 +275,23 @@ def test_trunk_broadcast_moe_output(gpu):
         got = model(ids)
         model.moe_forward = lambda block, x: x.mean(dims, keepdim=True).expand_as(x).contiguous()
         assert torch.equal(got, model(ids))
+
+
+@pytest.mark.parametrize("where,value", [("b_res", float("nan")), ("b_res", float("inf")), ("b_res", -float("inf")),
+                                         ("b_pre", float("nan")), ("b_post", float("inf")), ("B.weight", float("nan")),
+                                         ("X", float("nan")), ("X", float("inf"))])
+def test_mhc_not_finite(gpu, where, value):
+    """NaN and infinities come out of mhc_pre where the torch code has them: a NaN residual logit makes the
+    token's whole mix NaN, for the maximum and the clamped sums keep it."""
+    cfg = P.PrefillConfig(hidden=128, layers=1)
+    g = torch.Generator(device=gpu).manual_seed(7)
+    m = _fill(P._MHC(cfg).to(gpu), g, gpu, lambda n: {"A.weight": 0.02, "B.weight": 0.2}.get(n, 1.0))
+    norm = _fill(P._Norm(128).to(gpu), g, gpu, lambda n: 0.05)
+    X = torch.randn(1, 5, 4, 128, generator=g, device=gpu)
+    t = X if where == "X" else m.get_parameter(where).data
+    t.view(-1)[{"X": 900, "B.weight": 9 * cfg.mhc_rank + 2}.get(where, t.numel() // 2)] = value
+    with torch.no_grad():
+        x, (post, mix) = P._mhc_in(m, norm, X, X.pow(2).sum((2, 3)).view(-1), cfg, torch.float32)
+        xt, (postt, mixt) = P._mhc_in(m, norm, X, None, cfg, torch.float32)
+    for got, want, what in ((x, xt, "input"), (post, postt, "post"), (mix, mixt, "mix")):
+        torch.testing.assert_close(got.view(want.shape), want, rtol=1e-4, atol=1e-5, equal_nan=True, msg=what)
