@@ -4,6 +4,8 @@
 // tokens and hidden 1024) and, for the delta rule's chunk loop, some 400 launches per layer; here each
 // pass over the stream is one kernel, and the delta rule three. fp32 is computed in fp32 (MFMA forms
 // with fp32 operands), and values are rounded to the parameters' dtype where the torch code rounds.
+#include <type_traits>
+
 #include "q38moe_common.h"
 #include "q38moe_kernels.h"
 
@@ -669,6 +671,15 @@ __global__ __launch_bounds__(256) void qsa_prep_kernel(const void* __restrict__ 
   else st4_dt<BF16>(k_out, (t * KV + hd - H) * 64 + c, y);
 }
 
+// Zero in the place of every infinite bf16 value.
+__device__ __forceinline__ void drop_infinities(u32x4_t& v) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if ((v[i] & 0x7fffu) == 0x7f80u) v[i] &= 0xffff0000u;
+    if ((v[i] & 0x7fff0000u) == 0x7f800000u) v[i] &= 0xffffu;
+  }
+}
+
 // Attention of each 64-query block over its selected 64-key blocks, times sigmoid of the gate
 // (modeling:1143-1165): scores, softmax and sums in fp32. A workgroup takes the query block of one
 // sequence and key head for `hpw` of the query heads that share it; the key and value blocks lie in LDS
@@ -680,7 +691,10 @@ __global__ __launch_bounds__(256) void qsa_prep_kernel(const void* __restrict__ 
 // bf16: K Q^T by mfma_f32_16x16x32_bf16 (exact products, fp32 sums). The fp32 probabilities enter V^T P^T
 // as three bf16 parts by truncation, whose sum is the probability exactly (8 + 8 + 8 bits), so the
 // products with the bf16 values are exact too and only the fp32 sums round, as in an fp32 product; V
-// fragments come through the transposing LDS read, in the scores' key order.
+// fragments come through the transposing LDS read, in the scores' key order. An infinite value times a
+// part that is zero would be NaN where the fp32 product is infinite: a wave that sees a NaN repeats its
+// sums with infinities in the high part's product alone (the test costs 350.7 -> 352.3 us, launched alone
+// at the sizes below; 10.6 -> 10.8 at 1 x 192).
 // fp32: mfma_f32_16x16x4_f32 for both; the values take the keys' place in LDS after the scores, so a wave
 // runs one set of 16 queries (hpw = 2).
 // VALU-bound (exponentials and the three-way split, about 15 operations per score) next to 4 K MFMA
@@ -799,12 +813,12 @@ __global__ __launch_bounds__(512, 2) void qsa_attention_kernel(const void* __res
       __syncthreads();
     }
     f32x4_t o[4];
+    auto weigh_bf16 = [&](auto infinite) {
 #pragma unroll
-    for (int d = 0; d < 4; ++d) o[d] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+      for (int d = 0; d < 4; ++d) o[d] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      if (j >= nblk) break;
-      if (BF16) {
+      for (int j = 0; j < 8; ++j) {
+        if (j >= nblk) break;
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
           // Probabilities of keys 32 u + {4 lq + e, 16 + 4 lq + e}: high, middle and low 8 bits.
@@ -830,12 +844,28 @@ __global__ __launch_bounds__(512, 2) void qsa_attention_kernel(const void* __res
             const uint2 x = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_t)(uintptr_t)at));
             const uint2 y =
                 __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_t)(uintptr_t)(at + 16 * 128)));
-            const u32x4_t vf = {x.x, x.y, y.x, y.y};
+            u32x4_t vf = {x.x, x.y, y.x, y.y};
 #pragma unroll
-            for (int z = 0; z < 3; ++z) o[d] = mfma16x16x32(vf, part[z], o[d]);
+            for (int z = 0; z < 3; ++z) {
+              if (decltype(infinite)::value && z == 1) drop_infinities(vf);
+              o[d] = mfma16x16x32(vf, part[z], o[d]);
+            }
           }
         }
-      } else {
+      }
+    };
+    if constexpr (BF16) {
+      weigh_bf16(std::false_type{});
+      float any = 0.0f;  // NaN if a sum is (or sums of both infinities meet)
+#pragma unroll
+      for (int d = 0; d < 4; ++d) any += (o[d][0] + o[d][1]) + (o[d][2] + o[d][3]);
+      if (__builtin_expect(ballot64(any != any) != 0, 0)) weigh_bf16(std::true_type{});
+    } else {
+#pragma unroll
+      for (int d = 0; d < 4; ++d) o[d] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        if (j >= nblk) break;
 #pragma unroll
         for (int t = 0; t < 4; ++t)
 #pragma unroll

@@ -295,3 +295,26 @@ def test_mhc_not_finite(gpu, where, value):
         xt, (postt, mixt) = P._mhc_in(m, norm, X, None, cfg, torch.float32)
     for got, want, what in ((x, xt, "input"), (post, postt, "post"), (mix, mixt, "mix")):
         torch.testing.assert_close(got.view(want.shape), want, rtol=1e-4, atol=1e-5, equal_nan=True, msg=what)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_qsa_infinite_value(gpu, dtype):
+    """An infinite value comes through the weighted sum as an infinity, as in a product of fp32
+    probabilities, and not as the NaN of an infinity times a zero part of a probability."""
+    from q38.hip import ops
+    B, S, H, KV = 1, 192, 4, 2
+    g = torch.Generator(device=gpu).manual_seed(3)
+    r = lambda n, d=64: torch.randn(B, S, n, d, generator=g, device=gpu).to(dtype)
+    q, k, v, qg = r(H), r(KV), r(KV), r(H, 128)
+    v[0, 5, 0, 3], v[0, 9, 1, 40], v[0, 11, 1, 41] = float("inf"), -float("inf"), float("nan")
+    sel = torch.arange(3, device=gpu).expand(B, 3, 3).contiguous()
+    got = ops.qsa_attention(q, k, v, qg, sel, 0.125)
+    valid = torch.ones(3, 3, dtype=torch.bool, device=gpu).tril()
+    o = P.block_sparse_attention(*(t.transpose(1, 2) for t in (q, k, v)), sel, valid, 0.125)
+    want = o.transpose(1, 2).reshape(B, S, H * 64) * torch.sigmoid(qg[..., 64:].reshape(B, S, H * 64))
+    assert want.isinf().any() and want.isnan().any()
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isposinf(), want.isposinf())
+    assert torch.equal(got.isneginf(), want.isneginf())
+    ok = want.isfinite()
+    tol = 2e-5 if dtype == torch.float32 else 2**-7  # two bf16 roundings
+    torch.testing.assert_close(got[ok], want[ok], rtol=tol, atol=tol * 1e-1)
