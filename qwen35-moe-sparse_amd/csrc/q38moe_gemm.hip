@@ -864,8 +864,8 @@ hipError_t launch_down(const uint16_t* H, const int4* tiles, const int32_t* ntil
                        const uint16_t* ws_down, uint16_t* Y, int N, int K, int E,
                        hipStream_t stream) {
   if (use_gemm_wr(2 * K, tiles, max_mtiles, E))
-    return launch_down_wr(H, tiles, max_mtiles, M_dense, w_down, ws_down, Y, N, 2 * K, E, nullptr, nullptr, nullptr,
-                          stream);
+    return launch_down_wr(H, tiles, ntiles_dev, max_mtiles, M_dense, w_down, ws_down, Y, N, 2 * K, E, nullptr, nullptr,
+                          nullptr, stream);
   return down_impl(H, tiles, ntiles_dev, max_mtiles, M_dense, w_down, ws_down, Y, N, K, E, false, nullptr,
                    nullptr, nullptr, stream);
 }
@@ -890,8 +890,8 @@ hipError_t launch_down_fp8(const uint8_t* Hq, const int4* tiles, const int32_t* 
                            const float* s_sh_down, uint16_t* Y, int N, int K, int E,
                            hipStream_t stream) {
   if (use_gemm_wr(K, tiles, max_mtiles, E))
-    return launch_down_wr(Hq, tiles, max_mtiles, M_dense, wq_down, wq_sh_down, Y, N, K, E, a_scale, s_down, s_sh_down,
-                          stream);
+    return launch_down_wr(Hq, tiles, ntiles_dev, max_mtiles, M_dense, wq_down, wq_sh_down, Y, N, K, E, a_scale, s_down,
+                          s_sh_down, stream);
   return down_impl(Hq, tiles, ntiles_dev, max_mtiles, M_dense, wq_down, wq_sh_down, Y, N, K, E, true, a_scale,
                    s_down, s_sh_down, stream);
 }

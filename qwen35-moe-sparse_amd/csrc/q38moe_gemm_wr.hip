@@ -39,7 +39,8 @@ constexpr int WR_GROUPS = 65;                // 64 experts and the shared expert
 struct WrParams {
   const uint8_t* A;           // rows of KB bytes
   const int4* tiles;          // {group (E = shared expert), row0, rows, -} (group -1: unused); nullptr = M rows
-  int max_mtiles;
+  const int32_t* ntiles_dev;  // used entries of tiles
+  int max_mtiles;             // entries that tiles holds
   int64_t M;
   const uint8_t* W;           // [E, N, K]
   const uint8_t* Ws;          // shared expert [N, K]
@@ -106,9 +107,10 @@ __global__ __launch_bounds__(WR_THREADS, 2) void gemm_wr_kernel(WrParams p) {
   }
   __syncthreads();
   if (p.tiles != nullptr) {
+    const int used = load_uniform(p.ntiles_dev);  // its round trip overlaps the entries'
     for (int i = tid; i < p.max_mtiles; i += WR_THREADS) {
       const int4 t = p.tiles[i];
-      if (t.x >= 0 && t.x <= E) {
+      if (i < used && t.x >= 0 && t.x <= E) {
         atomicMin(&g_row0[t.x], t.y);
         atomicAdd(&g_rows[t.x], t.z);
       }
@@ -339,12 +341,12 @@ hipError_t launch_wr(const WrParams& p, int kb, hipStream_t stream) {
 
 bool gemm_wr_supported(int kb) { return kb == 256 || kb == 384 || kb == 512; }
 
-hipError_t launch_down_wr(const void* A, const int4* tiles, int max_mtiles, int64_t M_dense, const void* W,
-                          const void* Ws, uint16_t* C, int N, int kb, int E, const float* a_scale,
-                          const float* w_scale, const float* ws_scale, hipStream_t stream) {
+hipError_t launch_down_wr(const void* A, const int4* tiles, const int32_t* ntiles_dev, int max_mtiles,
+                          int64_t M_dense, const void* W, const void* Ws, uint16_t* C, int N, int kb, int E,
+                          const float* a_scale, const float* w_scale, const float* ws_scale, hipStream_t stream) {
   if (E > WR_GROUPS - 1 || N % 64 != 0) return hipErrorInvalidValue;
-  const WrParams p{static_cast<const uint8_t*>(A), tiles, max_mtiles, M_dense, static_cast<const uint8_t*>(W),
-                   static_cast<const uint8_t*>(Ws), C, N, E, a_scale, w_scale, ws_scale};
+  const WrParams p{static_cast<const uint8_t*>(A), tiles, ntiles_dev, max_mtiles, M_dense,
+                   static_cast<const uint8_t*>(W), static_cast<const uint8_t*>(Ws), C, N, E, a_scale, w_scale, ws_scale};
   return a_scale != nullptr ? launch_wr<true>(p, kb, stream) : launch_wr<false>(p, kb, stream);
 }
 

@@ -80,9 +80,9 @@ hipError_t launch_down(const uint16_t* H, const int4* tiles, const int32_t* ntil
 // Down-form products with the weights in registers (q38moe_gemm_wr.hip) for rows of kb bytes where
 // gemm_wr_supported(kb): launch_down and launch_down_fp8 (a_scale != nullptr) call it.
 bool gemm_wr_supported(int kb);
-hipError_t launch_down_wr(const void* A, const int4* tiles, int max_mtiles, int64_t M_dense, const void* W,
-                          const void* Ws, uint16_t* C, int N, int kb, int E, const float* a_scale,
-                          const float* w_scale, const float* ws_scale, hipStream_t stream);
+hipError_t launch_down_wr(const void* A, const int4* tiles, const int32_t* ntiles_dev, int max_mtiles,
+                          int64_t M_dense, const void* W, const void* Ws, uint16_t* C, int N, int kb, int E,
+                          const float* a_scale, const float* w_scale, const float* ws_scale, hipStream_t stream);
 
 // Four-wave bf16 grouped gate/up + SwiGLU (q38moe_gemm4w.hip): same arguments and results (up to fp32
 // summation order) as launch_gate_up, which calls it when gemm4w_supported(N, K, x_rows); x_rows

@@ -66,3 +66,24 @@ def test_down(gpu, fp8, E, k, T, K, N, sizes, shared):
             _assert_rounded(Y[st[e]:st[e] + ct[e]], H[st[e]:st[e] + ct[e]], W[e], allowance, f"expert {e}")
     if shared:
         _assert_rounded(Y[T * k:], H[T * k:], Ws, allowance, "shared expert")
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+def test_down_tile_count(gpu, fp8):
+    """Entries past *tile_count count for nothing, whatever a reused table still holds there."""
+    from q38.hip import ops
+    E, k, T, N, I = 6, 2, 800, 128, 256
+    g = torch.Generator().manual_seed(1)
+    idx = _routing(E, k, T, (0, 1, 300), g).to(gpu)
+    H, W = (torch.randn(*s, generator=g).to(torch.bfloat16).to(gpu) for s in ((T * k, I), (E, N, I)))
+    _, _, _, _, tiles, tc = ops.permute(idx, ops.histogram(idx, E), E)
+    if fp8:
+        (hq, hs), w = ops.quantize_rows(H), ops.quantize_rows(W)
+        wq = {"experts.down_proj": w, "shared_expert.down_proj.weight": tuple(t[0].contiguous() for t in w)}
+        run = lambda: ops.down_fp8(hq, hs, wq, tiles, tc, T, k)
+    else:
+        run = lambda: ops.down(H, W, tiles, tc, T, k)
+    expected = run()
+    assert int(tc) < len(tiles)
+    tiles[int(tc):] = tiles[0]
+    assert torch.equal(run(), expected)
