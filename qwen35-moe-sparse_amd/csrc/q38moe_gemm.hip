@@ -850,20 +850,35 @@ hipError_t launch_gate_up(const uint16_t* x, const int32_t* perm, const int4* ti
 }
 
 // Down-form launches with rows of kb bytes run with the weights in registers (q38moe_gemm_wr.hip) from
-// 160 rows per group on average (a tile table's routed and shared rows from its size, to 256), and for
-// every dense range. Below, a run covers one or two of its 64-row tiles per 256 KiB of weights and the
-// 256 x 256 units here are as fast or faster: h = 1024, I = 256, 64 experts + shared: 92 rows per group 17.9
-// here against 18.9 us there, 138 rows 18.4 / 18.8, 184 rows 21.1 / 18.6, 276 rows 43 / 22.5, 1510 rows
-// 75 / 61; e4m3 h = 2048, I = 512: 138 rows 30.4 / 33.3, 230 rows 75 / 42, 3025 rows 281 / 220 us.
-static bool use_gemm_wr(int kb, const int4* tiles, int max_mtiles, int E) {
-  return gemm_wr_supported(kb) && (tiles == nullptr || (int64_t)(max_mtiles - E) * BM >= (int64_t)160 * (E + 1));
+// 160 rows per group on average (a tile table's routed and shared rows from its size, to 256). Below, a
+// run covers one or two of its 64-row tiles per 256 KiB of weights and the 256 x 256 units here are as fast
+// or faster: h = 1024, I = 256, 64 experts + shared: 92 rows per group 17.9 here against 18.9 us there, 138
+// rows 18.4 / 18.8, 184 rows 21.1 / 18.6, 276 rows 43 / 22.5, 1510 rows 75 / 61; e4m3 h = 2048, I = 512:
+// 138 rows 30.4 / 33.3, 230 rows 75 / 42, 3025 rows 281 / 220 us.
+//
+// A dense range (a shared expert of another width than the routed ones) takes it too, except in two
+// places (gate/up and down of a shared expert, in us, here / there):
+// - up to 128 rows of 384 or 512 bytes and 448 to 768 columns: two column blocks' weights, loaded behind one
+//   another, are the whole time. N = 512, 512 bytes: 64 rows 19.3 / 20.2, 128 rows 21.0 / 21.7, 160 rows
+//   28.3 / 26.4; narrower and wider outputs gain or come out even (N = 256 17.9 / 16.6, N = 2048: 1 row
+//   39 / 36, 64 rows 36.0 / 36.6).
+// - two column blocks of which the second is half empty, with one or two tiles for each CU (N = 768, 512
+//   bytes: 8192 rows 36.8 / 38.7, 10240 rows 11 % behind, 16384 rows 40.9 / 41.7; but 5500 rows 38.5 / 36.1,
+//   24576 rows 14 % ahead). Other widths lie within 5 % either way there, by rows mod 256, or gain: N = 1024
+//   8192 rows 42.7 / 43.8, 16384 rows 48.7 / 47.3; N % 256 != 0 1.1 to 3 times as fast.
+static bool use_gemm_wr(int kb, const int4* tiles, int max_mtiles, int E, int64_t M_dense, int N) {
+  if (!gemm_wr_supported(kb)) return false;
+  if (tiles != nullptr) return (int64_t)(max_mtiles - E) * BM >= (int64_t)160 * (E + 1);
+  if (M_dense <= 128) return kb < 384 || N < 448 || N > 768;
+  const int64_t units = (M_dense + 63) / 64 * 2, cus = device_cus();
+  return N != 512 + 256 || 16 * units < 15 * cus || units > 2 * cus;
 }
 
 hipError_t launch_down(const uint16_t* H, const int4* tiles, const int32_t* ntiles_dev,
                        int max_mtiles, int64_t M_dense, const uint16_t* w_down,
                        const uint16_t* ws_down, uint16_t* Y, int N, int K, int E,
                        hipStream_t stream) {
-  if (use_gemm_wr(2 * K, tiles, max_mtiles, E))
+  if (use_gemm_wr(2 * K, tiles, max_mtiles, E, M_dense, N))
     return launch_down_wr(H, tiles, ntiles_dev, max_mtiles, M_dense, w_down, ws_down, Y, N, 2 * K, E, nullptr, nullptr,
                           nullptr, stream);
   return down_impl(H, tiles, ntiles_dev, max_mtiles, M_dense, w_down, ws_down, Y, N, K, E, false, nullptr,
@@ -889,7 +904,7 @@ hipError_t launch_down_fp8(const uint8_t* Hq, const int4* tiles, const int32_t* 
                            const uint8_t* wq_down, const float* s_down, const uint8_t* wq_sh_down,
                            const float* s_sh_down, uint16_t* Y, int N, int K, int E,
                            hipStream_t stream) {
-  if (use_gemm_wr(K, tiles, max_mtiles, E))
+  if (use_gemm_wr(K, tiles, max_mtiles, E, M_dense, N))
     return launch_down_wr(Hq, tiles, ntiles_dev, max_mtiles, M_dense, wq_down, wq_sh_down, Y, N, K, E, a_scale, s_down,
                           s_sh_down, stream);
   return down_impl(Hq, tiles, ntiles_dev, max_mtiles, M_dense, wq_down, wq_sh_down, Y, N, K, E, true, a_scale,

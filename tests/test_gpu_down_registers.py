@@ -87,3 +87,38 @@ def test_down_tile_count(gpu, fp8):
     assert int(tc) < len(tiles)
     tiles[int(tc):] = tiles[0]
     assert torch.equal(run(), expected)
+
+
+@pytest.mark.parametrize("h,Is,rows", [
+    (320, 128, (1, 64, 65, 129)),         # part of one column block
+    (576, 256, (1, 64, 128, 129, 200)),   # a second block of one wave; both sides of 128 rows
+    (768, 192, (128, 129, 7616, 7617, 16384, 16385)),  # both sides of one and two tiles per CU (256 CUs)
+    (1024, 256, (1, 65, 5003))])
+def test_down_dense(gpu, h, Is, rows):
+    """Dense ranges (a shared expert by itself), from one row on, at the bar of test_down."""
+    from q38.hip import ops
+    g = torch.Generator().manual_seed(h)
+    wg, wu, wd = ((torch.randn(*s, generator=g) * 0.05).to(torch.bfloat16).to(gpu) for s in ((Is, h), (Is, h), (h, Is)))
+    ptr = lambda t: t.data_ptr()
+    for T in rows:
+        x = torch.randn(T, h, generator=g).to(torch.bfloat16).to(gpu)
+        H, out = torch.empty(T, Is, dtype=torch.bfloat16, device=gpu), torch.empty_like(x)
+        rc = ops.lib.q38moe_shared_expert(ptr(x), ptr(wg), ptr(wu), ptr(wd), ptr(H), ptr(out), T, h, Is, ops.BF16,
+                                          torch.cuda.current_stream().cuda_stream)
+        assert rc == 0
+        _assert_rounded(out, H, wd, 2.0**-20, f"{T} rows")
+
+
+@pytest.mark.parametrize("T", [1, 130, 3000])
+def test_down_dense_in_block(gpu, T):
+    """The dense range of a block with 64 experts: with routed experts that give zeros and a shared gate of
+    1/2, the block's output is half the shared expert's, bit for bit."""
+    from q38.hip import ops
+    E, k, h, I, Is = 64, 2, 512, 128, 256
+    g = torch.Generator().manual_seed(T)
+    r = lambda *s: (torch.randn(*s, generator=g) * 0.05).to(torch.bfloat16).to(gpu)
+    x, wr, wgu, wg, wu, wd = r(T, h) * 20, r(E, h), r(E, 2 * I, h), r(Is, h), r(Is, h), r(h, Is)
+    wdn, gate = torch.zeros(E, h, I, dtype=torch.bfloat16, device=gpu), torch.zeros(1, h, dtype=torch.bfloat16, device=gpu)
+    with torch.inference_mode():
+        out = ops.block_forward(x, wr, wgu, wdn, wg, wu, wd, gate, k)
+        assert torch.equal(out, ops.shared_expert(x, wg, wu, wd) * 0.5)
