@@ -165,10 +165,14 @@ def _qsa64(m, sel, x, cos, sin, cfg):
     (1, 64, 2, 2, 8, 0.25, 1.0),     # one block, one head per workgroup
     (2, 320, 6, 2, 3, 0.5, 1.0),     # fewer blocks than the sequence has, an odd number of heads per key head
     (1, 1024, 38, 2, 8, 0.25, 1.0),
-    (4, 1088, 10, 1, 8, 1.0, 6.0)])  # four heads per workgroup (bf16), a partial set of them; peaked softmax
+    (4, 1088, 10, 1, 8, 1.0, 6.0),   # one key head, all features rotated; peaked softmax
+    (4, 1088, 38, 2, 8, 0.25, 6.0)])  # four heads per workgroup (bf16), three in the last
 def test_qsa(gpu, dtype, B, S, H, KV, blocks, rotary, spread):
     """qsa_prep and qsa_attention inside the mixer, on the key blocks the indexer selects."""
     cfg = P.PrefillConfig(hidden=256, layers=1, heads=H, kv_heads=KV, qsa_blocks=blocks, partial_rotary=rotary)
+    if H == 38 and B == 4:  # launch_qsa_attention's rule
+        sets = -(-(H // KV) // 4)
+        assert B * (S // 64) * KV * sets >= 2 * torch.cuda.get_device_properties(gpu).multi_processor_count
     g = torch.Generator(device=gpu).manual_seed(S + H)
     m = _fill(P._Attention(cfg).to(gpu), g, gpu, lambda n: spread if "norm" in n else 0.06).to(dtype)
     ix = _fill(P._Indexer(cfg).to(gpu), g, gpu, lambda n: 0.1).to(dtype)
