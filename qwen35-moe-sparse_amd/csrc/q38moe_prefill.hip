@@ -1,9 +1,10 @@
-// Kernels of the packed prefill's trunk around the MoE block: the mHC residual stream and the Gated
-// DeltaNet token mixer and the QSA attention (modeling_qwen3_8_moe.py:994-1031, 132-349, 464-577, 1117-1165). As torch operations both
-// are chains of passes over large fp32 tensors (the four-branch stream alone is 268 MB at 4 x 4096
-// tokens and hidden 1024) and, for the delta rule's chunk loop, some 400 launches per layer; here each
-// pass over the stream is one kernel, and the delta rule three. fp32 is computed in fp32 (MFMA forms
-// with fp32 operands), and values are rounded to the parameters' dtype where the torch code rounds.
+// Kernels of the packed prefill's trunk around the MoE block: the mHC residual stream
+// (modeling_qwen3_8_moe.py:994-1031), the Gated DeltaNet token mixer (132-349, 464-577) and the QSA
+// attention (1117-1165). As torch operations these are chains of passes over large fp32 tensors (the
+// four-branch stream alone is 268 MB at 4 x 4096 tokens and hidden 1024) and, for the delta rule's chunk
+// loop, some 400 launches per layer. Here each pass over the stream is one kernel, the delta rule with its
+// gated norm three, and the attention one. fp32 is computed in fp32 (MFMA forms with fp32 operands), and
+// values are rounded to the parameters' dtype where the torch code rounds.
 #include <type_traits>
 
 #include "q38moe_common.h"

@@ -10,12 +10,13 @@ parameter names follow the reference state dict (``model.layers.{i}.linear_attn.
 Per layer (modeling:1259-1275): mHC pre-mix of the 4-way residual stream (fp32), zero-centred
 RMSNorm, the token mixer (Gated DeltaNet, or QSA sparse attention on every 4th layer), mHC post-mix;
 then the same around the MoE block; after layer 0 the N-gram embedding adds its gated delta. The
-token mixers are torch code on the GPU (hipBLASLt GEMMs); only the MoE runs on this library's
-kernels.
+projections are torch products on the GPU (hipBLASLt GEMMs). The MoE block and, for the forwards that
+``_native_trunk`` takes, the mHC stream, the delta rule and the sparse attention run on this library's
+kernels; the torch code here is what the others run and what the kernels are tested against.
 
 Numerics follow the reference op for op where a rounding point is visible (bf16 projections, fp32
-mHC stream, fp32 delta-rule state, bf16 gating products). Two restatements differ in form, not in
-math: the causal depthwise convolution is an explicit fp32 shift-and-add (modeling:184-205 uses
+mHC stream, fp32 delta-rule state, bf16 gating products). Two restatements of the torch code differ in
+form, not in math: the causal depthwise convolution is an explicit fp32 shift-and-add (modeling:184-205 uses
 conv1d), and QSA attention gathers each query block's selected key blocks and runs dense fp32
 attention on them, which equals the reference's masked attention over the full sequence
 (modeling:1143-1158).
@@ -574,6 +575,7 @@ def _native_trunk(M, cfg, ids):
         return False
     if ids.device.index != torch.cuda.current_device() or ids.numel() >= 2 ** 24:  # one block of 256 per token
         return False
+    # mhc_pre's limits; the rank, hidden / 8, keeps models above hidden 1024 on the torch code.
     if cfg.hidden % 64 or cfg.hidden > 2048 or cfg.mhc_rank % 4 or cfg.mhc_rank > 128:
         return False
     if torch.is_grad_enabled() or torch.is_autocast_enabled("cuda"):

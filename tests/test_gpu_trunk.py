@@ -83,6 +83,18 @@ def test_mhc_sublayer(gpu, dtype, B, S, h):
     assert torch.allclose(ssq.double(), X.double().pow(2).sum((2, 3)).view(-1), rtol=1e-6)
 
 
+class _Rank128(P.PrefillConfig):
+    mhc_rank = 128
+
+
+@pytest.mark.parametrize("B,S,h", [(1, 5, 1088), (1, 3, 1472), (2, 33, 2048),
+                                   (1, 8193, 1792)])  # 16 tokens per block, the last one with one
+def test_mhc_wide(gpu, monkeypatch, B, S, h):
+    """Hidden sizes above 1024 at a rank the kernel takes (PrefillConfig's own, hidden / 8, is above it)."""
+    monkeypatch.setattr(P, "PrefillConfig", _Rank128)
+    test_mhc_sublayer(gpu, torch.bfloat16, B, S, h)
+
+
 def _delta64(m, x, cfg):
     """The DeltaNet mixer in float64, token by token (modeling:352-413, 464-577)."""
     w = {n: p.detach().double() for n, p in m.named_parameters()}
