@@ -587,7 +587,8 @@ def _native_trunk(M, cfg, ids):
     dt = M.embed_tokens.weight.dtype
     if dt not in (torch.bfloat16, torch.float32):
         return False
-    return all(p.dtype == dt and p.device == ids.device and p.is_contiguous() and p.data_ptr() % 16 == 0
+    gpu = ids.get_device()
+    return all(p.dtype == dt and p.get_device() == gpu and p.is_contiguous() and p.data_ptr() % 16 == 0
                and type(p) in (torch.Tensor, nn.Parameter) for p in M.parameters())
 
 
@@ -615,7 +616,9 @@ def _mhc_out(X, y, state, ssq):
     B, S, n, h = X.shape
     if y.dtype not in (torch.bfloat16, torch.float32):
         y = y.float()
-    y = y.expand(B, S, h).reshape(B * S, h).contiguous()
+    if y.shape != (B, S, h):
+        y = y.expand(B, S, h)
+    y = y.reshape(B * S, h).contiguous()
     if y.data_ptr() % 16:  # the MoE callable may return a view of a buffer of its own
         y = y.clone()
     ops.mhc_update(ops.MHC_POST, X.view(B * S, n, h), y, ssq, *state)
