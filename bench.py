@@ -311,7 +311,7 @@ def copy_probe(mib):
 
 def prefill_bench(args):
     """Workload c5: the packed no-cache prefill of a 12-layer random-init Q38 model (q38.prefill)
-    on 4 x 4096 tokens, the fused HIP MoE block in every layer; the token mixers are torch code.
+    on 4 x 4096 tokens, the fused HIP MoE block in every layer and the trunk on its own kernels around torch's projections.
     Reports whole-model tokens/s, the share of the 12 MoE blocks, and a bounded CPU sample of the
     same restatement (CPU oracle in place of the HIP blocks)."""
     import torch

@@ -699,7 +699,7 @@ __device__ __forceinline__ void drop_infinities(u32x4_t& v) {
 // fp32: mfma_f32_16x16x4_f32 for both; the values take the keys' place in LDS after the scores, so a wave
 // runs one set of 16 queries (hpw = 2).
 // VALU-bound (exponentials and the three-way split, about 15 operations per score) next to 4 K MFMA
-// cycles per 16 queries: 385-400 us at 4 x 4096 tokens, 38 heads on 2, 8 blocks (the torch operations,
+// cycles per 16 queries: 385-400 us in a prefill of 4 x 4096 tokens, 38 heads on 2, 8 blocks (the torch operations,
 // fp32 products on gathered blocks with 2.5 GB of scores in memory, about 5 ms).
 template <bool BF16>
 __global__ __launch_bounds__(512, 2) void qsa_attention_kernel(const void* __restrict__ q, const void* __restrict__ k,

@@ -986,7 +986,9 @@ __global__ __launch_bounds__(NARROW_WAVES * 64) void route_narrow_kernel(
 // on 256 CUs; above, a second round would cost more than the 64-token blocks: T = 5003 17.8 against 17.5
 // us at h = 1024). Two groups of 16 per block for up to 8192 tokens measured 17.1 against 17.5 us at
 // h = 1024, 20.1 against 23.2 at 2048, but the permutation then reads up to four times the histogram
-// rows, which took that back. h % 512: whole MFMA steps per wave.
+// rows, which took that back (at T = 4096 its 256 rows cost 7.3 against 5.7 us at h = 1024, 8.4 against 6.6
+// at 2048, where the router gains 5.8 and 9.3). h % 512: whole MFMA steps per wave; other widths run the
+// 64-token blocks at every T.
 int route_tokens_per_row(int64_t T, int h) {
   const bool narrow = h % 512 == 0 && (T + NARROW_TOKENS - 1) / NARROW_TOKENS <= device_cus();
   return narrow ? NARROW_TOKENS : ROUTE_TOKENS;
