@@ -616,7 +616,7 @@ def _mhc_out(X, y, state, ssq):
     B, S, n, h = X.shape
     if y.dtype not in (torch.bfloat16, torch.float32):
         y = y.float()
-    if y.shape != (B, S, h):
+    if y.numel() != B * S * h:  # broadcast over tokens or features
         y = y.expand(B, S, h)
     y = y.reshape(B * S, h).contiguous()
     if y.data_ptr() % 16:  # the MoE callable may return a view of a buffer of its own
