@@ -421,9 +421,9 @@ def _delta_net(m, x, cfg, native=False):
             and B * S * (2 * nk + nv) < 2 ** 31):
         from .hip import ops
 
-        o = ops.gdn_delta(ops.gdn_conv(qkv, m.conv1d.weight), F.linear(x, m.in_proj_b.weight),
+        o = ops.gdn_delta(ops.gdn_conv(qkv, _aligned(m.conv1d.weight)), F.linear(x, m.in_proj_b.weight),
                           F.linear(x, m.in_proj_a.weight), m.A_log, m.dt_bias, F.linear(x, m.in_proj_z.weight),
-                          m.norm.weight, nk, nv, cfg.rms_eps)
+                          _aligned(m.norm.weight), nk, nv, cfg.rms_eps)
         return F.linear(o, m.out_proj.weight)
     # Causal depthwise convolution (kernel K, left zero padding) in fp32, then SiLU in x.dtype.
     w = m.conv1d.weight[:, 0, :].float()
@@ -478,7 +478,7 @@ def _qsa(m, ix, x, cos, sin, cfg, native=False):
             and B * S * (H + KV) < 2 ** 31):
         from .hip import ops
 
-        q, k = ops.qsa_prep(qg, k, m.q_norm.weight, m.k_norm.weight, cos, sin, cfg.rms_eps)
+        q, k = ops.qsa_prep(qg, k, _aligned(m.q_norm.weight), _aligned(m.k_norm.weight), cos, sin, cfg.rms_eps)
         sel, _ = _qsa_select(ix, x, cos, sin, cfg)
         return F.linear(ops.qsa_attention(q, k, v, qg, sel.contiguous(), hd ** -0.5), m.o_proj.weight)
     q, gate = qg[..., :hd], qg[..., hd:].reshape(B, S, H * hd)
@@ -565,9 +565,8 @@ def _mhc_post(X, y, state):
 
 def _native_trunk(M, cfg, ids):
     """True when the trunk's own kernels (q38.hip.ops.mhc_*, gdn_*, qsa_*) take this forward: tokens and parameters
-    plain tensors on the current GPU, parameters all bf16 or all fp32, contiguous and on 16-byte boundaries (views
-    into a flat buffer need not be), no gradient, autocast, tracing or function transform in force, and the shapes
-    they are built for. Otherwise the torch code runs.
+    plain tensors on the current GPU, parameters all bf16 or all fp32 and contiguous, no gradient, autocast,
+    tracing or function transform in force, and the shapes they are built for. Otherwise the torch code runs.
     Gradients by mode and not by the parameters: the MoE callable may hold parameters of its own."""
     from torch.autograd import forward_ad
 
@@ -588,8 +587,14 @@ def _native_trunk(M, cfg, ids):
     if dt not in (torch.bfloat16, torch.float32):
         return False
     gpu = ids.get_device()
-    return all(p.dtype == dt and p.get_device() == gpu and p.is_contiguous() and p.data_ptr() % 16 == 0
+    return all(p.dtype == dt and p.get_device() == gpu and p.is_contiguous()
                and type(p) in (torch.Tensor, nn.Parameter) for p in M.parameters())
+
+
+def _aligned(t):
+    """t, or a copy of it where t does not start on the 16-byte boundary that the kernels' entry points ask for
+    (a view into a flat buffer)."""
+    return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
 def _mhc_in(m, norm, X, ssq, cfg, dt):
@@ -603,7 +608,7 @@ def _mhc_in(m, norm, X, ssq, cfg, dt):
     B, S, n, h = X.shape
     z0 = F.linear(X.view(B * S, n * h), m.A.weight.float())
     x, post, P = ops.mhc_pre(X.view(B * S, n, h), ssq, z0, m.B.weight, m.b_pre, m.b_post, m.b_res, m.alphas,
-                             norm.weight, cfg.mhc_iters, cfg.rms_eps)
+                             _aligned(norm.weight), cfg.mhc_iters, cfg.rms_eps)
     return x.view(B, S, h), (post, P)
 
 
@@ -618,9 +623,7 @@ def _mhc_out(X, y, state, ssq):
         y = y.float()
     if y.numel() != B * S * h:  # broadcast over tokens or features
         y = y.expand(B, S, h)
-    y = y.reshape(B * S, h).contiguous()
-    if y.data_ptr() % 16:  # the MoE callable may return a view of a buffer of its own
-        y = y.clone()
+    y = _aligned(y.reshape(B * S, h).contiguous())  # the MoE callable may return a view of a buffer of its own
     ops.mhc_update(ops.MHC_POST, X.view(B * S, n, h), y, ssq, *state)
     return X
 
